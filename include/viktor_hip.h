@@ -495,6 +495,14 @@ int vk_strict_identity(const uint8_t *calls, const int64_t *call_off, const int3
                        float *reward, int32_t *edit_distance, int32_t *scored_errors, void *stream);
 
 /*
+ * The base strings of n_rows rows of output tokens [n_rows, T] (viktor/tokenizer.py's decode: up to the first eos,
+ * ids clamped into the vocabulary): row c's bytes to out[c * T * k ..], len[c] of them. table [vocab, k + 1] uint8:
+ * each token's bytes (k at most) and, in the last column, how many it has (0 for special tokens).
+ */
+int vk_tokens_to_bases(const int64_t *tokens, int32_t n_rows, int32_t T, const uint8_t *table, int32_t vocab, int32_t k,
+                       int32_t eos, uint8_t *out, int32_t *len, void *stream);
+
+/*
  * The encoder (frames producer): the Dorado SUP conv stack + sliding-window DeepNorm transformer of
  * viktor/encoder.py:43-192, which the reference runs on koi (viktor/csrc/koi_tx.cpp:253-414: koi_vcs_tx_cnn,
  * koi_qkv_rotary + koi_vcs_attn, koi_linear, koi_rmsnorm_residual, koi_mm_swiglu).

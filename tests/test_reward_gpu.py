@@ -98,3 +98,36 @@ def test_rewards_from_tokens_equal_rewards_from_strings():
     assert np.array_equal(dev_res["reward"].double().cpu().numpy().reshape(-1, G), host)
     for i, c in enumerate(calls):
         assert abs(host.reshape(-1)[i] - R.strict_identity_ref(c, labels[i // G], weights[i // G] > 0)[0]) < 1e-6
+
+
+@pytest.mark.parametrize("m", [1, 7, 8, 9, 511, 512, 513, 1023, 1024, 1025, 2500, 4095])
+def test_strict_identity_at_the_edges_of_lanes_and_wavefronts(m):
+    """Labels that end on or beside a lane's 8 rows and a wavefront's 512, calls beside a block of 64 columns, up to the
+    longest of both."""
+    rng = np.random.default_rng(m)
+    labels = ["".join(rng.choice(list("ACGT"), m)), "".join(rng.choice(list("AC"), max(1, m - 5)))]
+    scored = [rng.random(len(l)) > 0.3 for l in labels]
+    calls = ["".join(rng.choice(list("ACGT"), n)) for n in (0, 1, 2, 63, 64, 65, 129)]
+    calls += [_mutate(rng, labels[0], 0.1), _mutate(rng, labels[1], 0.4)]
+    if m in (512, 4095):
+        calls.append("".join(rng.choice(list("ACGT"), 8192)))
+    _check(calls, labels, scored, [i % 2 for i in range(len(calls))])
+
+
+@pytest.mark.parametrize("k,T", [(1, 1), (1, 1023), (1, 1024), (1, 1025), (4, 3), (4, 2050)])
+def test_token_rows_at_the_edges_of_a_pass(k, T):
+    """Rows that end on or beside a workgroup's pass of 1024 tokens, EOS at a pass's first and last token, ids outside
+    the vocabulary (clamped)."""
+    rng = np.random.default_rng(T)
+    tok = KmerTokenizer(k)
+    rows = torch.tensor(rng.integers(0, tok.vocab_size, (8, T)), dtype=torch.long)
+    rows[rows == 2] = 3
+    for b, at in enumerate((0, T // 2, T - 1, 1023, 1024)):
+        if at < T:
+            rows[b, at] = 2
+    rows[6, 0], rows[7, -1] = -5, 10 ** 6
+    got, off, lens, longest = RW.calls_from_tokens(rows.to(DEV), tok)
+    got, off, lens = got.cpu().numpy(), off.cpu().numpy(), lens.cpu().numpy()
+    want = [tok.decode(r.tolist()) for r in rows.clamp(0, tok.vocab_size - 1)]
+    assert [bytes(got[o:o + n]).decode() for o, n in zip(off, lens)] == want
+    assert longest == max(len(w) for w in want)

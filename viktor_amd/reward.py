@@ -3,7 +3,7 @@
 Reference: scripts/gspo.py:86-89 (strict_identity), 446 (the reward of a rollout), scripts/train.py:170-188
 (ref_errors, the edlib NW path's error positions), scripts/evaluate.py:30 (EMPTY_MAX). The reference runs
 edlib on the host, one call after another; here one kernel scores every call of a rollout at once
-(vk_strict_identity: one wavefront per call, anti-diagonal edit-distance DP in LDS).
+(vk_strict_identity: the edit-distance DP as a systolic array, 512 label rows per wavefront).
 
 The alignment path behind the error positions: at every cell the first optimal predecessor in the order
 diagonal, deletion, insertion. edlib's own traceback order is not available here; the edit distance, and
@@ -19,6 +19,7 @@ from . import _lib
 from ._lib import call, ptr, require_device
 from .tokenizer import EOS, N_SPECIAL
 
+MAX_CALL = 8192  # the longest call vk_strict_identity takes
 EMPTY_MAX = 4  # scripts/evaluate.py:30: a window without DNA scores 1 for a call of at most this many bases
 
 
@@ -32,21 +33,38 @@ def _pack(strings: Sequence[bytes], device):
             torch.tensor(lens, dtype=torch.int32).to(device), max(lens) if lens else 0)
 
 
+def _upload(arrays, device):
+    """Host arrays as device tensors of one upload (8-byte aligned slices of one buffer)."""
+    sizes = [-(-a.nbytes // 8) * 8 for a in arrays]
+    host = np.zeros(max(sum(sizes), 8), dtype=np.uint8)
+    o = 0
+    spans = []
+    for a, n in zip(arrays, sizes):
+        host[o:o + a.nbytes] = a.reshape(-1).view(np.uint8)
+        spans.append((o, a.nbytes, getattr(torch, a.dtype.name)))
+        o += n
+    dev = torch.from_numpy(host).to(device)
+    return [dev[o:o + n].view(dt) for o, n, dt in spans]
+
+
 def _run(call_data, call_off, call_len, max_call, refs: Sequence[str], scored: Sequence[np.ndarray], ref_of_call,
          device, empty_max):
     ref_b = [r.encode() for r in refs]
-    ref_data, ref_off, ref_len, max_ref = _pack(ref_b, device)
     sc = [np.asarray(s, dtype=bool).astype(np.uint8) for s in scored]
     assert all(len(s) == len(r) for s, r in zip(sc, ref_b)), "strict_identity: a scored mask per label base"
-    sc_data = torch.from_numpy(np.concatenate(sc) if sum(len(s) for s in sc) else np.zeros(1, np.uint8)).to(device)
+    lens = np.array([len(r) for r in ref_b], dtype=np.int32)
+    off = np.concatenate([[0], np.cumsum(lens[:-1], dtype=np.int64)])[:len(lens)].astype(np.int64)
+    data = np.frombuffer(b"".join(ref_b) or b"\0", dtype=np.uint8)
+    mask = np.concatenate([*sc, np.zeros(0 if lens.sum() else 1, np.uint8)])
+    ref_off, ref_len, roc, ref_data, sc_data = _upload([off, lens, np.asarray(ref_of_call, dtype=np.int32), data, mask],
+                                                       device)
     n = call_len.shape[0]
-    roc = torch.as_tensor(ref_of_call, dtype=torch.int32).to(device)
     reward = torch.empty(n, dtype=torch.float32, device=device)
     dist = torch.empty(n, dtype=torch.int32, device=device)
     errs = torch.empty(n, dtype=torch.int32, device=device)
     call("vk_strict_identity", ptr(call_data), ptr(call_off), ptr(call_len), ptr(ref_data), ptr(ref_off),
-         ptr(ref_len), ptr(sc_data), ptr(roc), n, len(refs), max_ref, max_call, float(empty_max), ptr(reward),
-         ptr(dist), ptr(errs), _lib.stream_handle())
+         ptr(ref_len), ptr(sc_data), ptr(roc), n, len(refs), int(lens.max()) if len(lens) else 0, max_call,
+         float(empty_max), ptr(reward), ptr(dist), ptr(errs), _lib.stream_handle())
     return {"reward": reward, "edit_distance": dist, "scored_errors": errs}
 
 
@@ -69,37 +87,42 @@ def gspo_rewards(calls: List[str], labels: List[str], weights: List[np.ndarray],
     return res["reward"].double().cpu().numpy().reshape(-1, G)
 
 
+def _bases(tokens: torch.Tensor, tokenizer):
+    """The base strings of output tokens [N, T] on the device (vk_tokens_to_bases): rows [N, T k] uint8 and their
+    lengths [N] int32. No host synchronisation."""
+    N, T = tokens.shape
+    V, k = tokenizer.vocab_size, tokenizer.k
+    strings = [b"" if t < N_SPECIAL else tokenizer.strings[t].encode() for t in range(V)]
+    host = b"".join(s.ljust(k, b"\0") + bytes([len(s)]) for s in strings)
+    table = torch.from_numpy(np.frombuffer(host, dtype=np.uint8).copy()).to(tokens.device)
+    tokens = tokens.long().contiguous()
+    rows = torch.empty(N, T * k, dtype=torch.uint8, device=tokens.device)
+    lens = torch.empty(N, dtype=torch.int32, device=tokens.device)
+    call("vk_tokens_to_bases", ptr(tokens), N, T, ptr(table), V, k, EOS, ptr(rows), ptr(lens), _lib.stream_handle())
+    return rows, lens
+
+
 def calls_from_tokens(tokens: torch.Tensor, tokenizer):
     """Device base strings of the engine's output tokens [N, T] (int64): the tokenizer's decode on the device
     (stops at the first EOS, skips PAD and BOS; a token writes its k-mer or tail). Returns (bytes [total] uint8,
     offsets [N] int64, lengths [N] int32, max length)."""
-    dev = tokens.device
-    V, k = tokenizer.vocab_size, tokenizer.k
-    table = torch.zeros(V, k, dtype=torch.uint8)
-    tlen = torch.zeros(V, dtype=torch.int64)
-    for t in range(N_SPECIAL, V):
-        s = tokenizer.strings[t].encode()
-        table[t, :len(s)] = torch.tensor(list(s), dtype=torch.uint8)
-        tlen[t] = len(s)
-    table, tlen = table.to(dev), tlen.to(dev)
-    tok = tokens.clamp(0, V - 1)
-    before_eos = torch.cumsum((tok == EOS).to(torch.int32), 1) == 0
-    n_bases = tlen[tok] * before_eos                      # [N, T] bases each token writes
-    lengths = n_bases.sum(1)
-    offsets = torch.cumsum(lengths, 0) - lengths
-    pos = offsets[:, None] + torch.cumsum(n_bases, 1) - n_bases  # first byte of each token
-    total = int(lengths.sum())
-    out = torch.zeros(max(total, 1), dtype=torch.uint8, device=dev)
-    for i in range(k):  # byte i of every token that has one
-        keep = n_bases > i
-        out[(pos + i)[keep]] = table[tok, i][keep]
-    return out, offsets, lengths.to(torch.int32), int(lengths.max()) if lengths.numel() else 0
+    rows, lens = _bases(tokens, tokenizer)
+    offsets = torch.cumsum(lens.long(), 0) - lens
+    out = rows[torch.arange(rows.shape[1], device=rows.device) < lens[:, None]]
+    if out.numel() == 0:
+        out = torch.zeros(1, dtype=torch.uint8, device=rows.device)
+    return out, offsets, lens, int(lens.max()) if lens.numel() else 0
 
 
 def gspo_rewards_from_tokens(tokens: torch.Tensor, tokenizer, labels: List[str], weights: List[np.ndarray], G: int,
                              empty_max=EMPTY_MAX):
     """The rollout's rewards straight from the engine's device output (no host decode): tokens [windows * G, T];
     returns the device dict of strict_identity (reward [windows * G] fp32)."""
-    data, off, lens, max_call = calls_from_tokens(tokens, tokenizer)
-    return _run(data, off, lens, max_call, labels, [np.asarray(w) > 0 for w in weights],
-                [i // G for i in range(tokens.shape[0])], tokens.device, empty_max)
+    require_device(tokens, "gspo_rewards_from_tokens")
+    rows, lens = _bases(tokens, tokenizer)
+    N, width = rows.shape
+    # rows longer than the kernel's longest call: only then the lengths are read back
+    longest = width if width <= MAX_CALL else int(lens.max())
+    off = torch.arange(N, device=rows.device) * width
+    return _run(rows, off, lens, longest, labels, [np.asarray(w) > 0 for w in weights], np.arange(N) // G,
+                tokens.device, empty_max)
