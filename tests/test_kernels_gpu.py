@@ -127,6 +127,20 @@ def test_linear(M, N, K):
     assert torch.allclose(y32.cpu().double(), ref, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("N", [8, 392, 424])
+def test_swiglu_kept_rows_ragged_columns(N):
+    """The kept gate | up rows at N that is no multiple of a wavefront's 32 columns: nothing is stored past a half of a
+    row or past the last row."""
+    g = gen(N)
+    M, K = 4097, 128
+    x = to_dev(R.bf(torch.randn(M, K, generator=g)), BF)
+    w = to_dev(R.bf(torch.randn(2 * N, K, generator=g) / math.sqrt(K)), BF)
+    whole = torch.full((M + 1, 2 * N), 7.0, dtype=BF, device=DEV)
+    ops.linear(x, w, swiglu=True, gu_out=whole[:M])
+    assert torch.equal(whole[:M], torch.cat([ops.linear(x, w[:N].contiguous()), ops.linear(x, w[N:].contiguous())], 1))
+    assert bool((whole[M] == 7.0).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(4099, 1536, 512), (8192, 520, 512), (4608, 512, 1536), (5000, 3072, 1024)])
 def test_linear_large_m_tile_shapes_same_bits(M, N, K):
     """Large M: bf16 outputs run 256 x 256 tiles, fp32 outputs at K < 1024 the 256 x 128 tiles; both accumulate

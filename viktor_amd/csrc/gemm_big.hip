@@ -522,7 +522,7 @@ __global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
         // 0.007% of the outputs then differ from the division's by one bf16 ulp
         // qa.raw: the gate | up product rows [M, 2 N] as the plain product stores them (the backward's operand)
         const int64_t grow = qrow0 + 16 * j + fr;
-        const bool keep = qa.raw != nullptr && grow < M && qcol0 < N;
+        const bool keep = qa.raw != nullptr && grow < M;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           float o[4], gt4[4], up4[4];
@@ -535,7 +535,7 @@ __global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
             o[e] = round_bf(gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt))) * up;
           }
           *reinterpret_cast<u32x2 *>(rowp + (16 * i + 4 * fg) * 2) = u32x2{pack_bf(o[0], o[1]), pack_bf(o[2], o[3])};
-          if (keep) {
+          if (keep && qcol0 + 16 * i + 4 * fg < N) {  // (N % 8 == 0: 4 columns are all inside or all outside)
             bf16_t *gr = qa.raw + grow * (2 * static_cast<int64_t>(N)) + qcol0 + 16 * i + 4 * fg;
             *reinterpret_cast<u32x2 *>(gr) = u32x2{pack_bf(gt4[0], gt4[1]), pack_bf(gt4[2], gt4[3])};
             *reinterpret_cast<u32x2 *>(gr + N) = u32x2{pack_bf(up4[0], up4[1]), pack_bf(up4[2], up4[3])};
