@@ -141,6 +141,54 @@ def test_swiglu_kept_rows_ragged_columns(N):
     assert bool((whole[M] == 7.0).all())
 
 
+@pytest.mark.parametrize("M,K", [(4096, 64), (4223, 128), (4097, 192), (4352, 320)])
+def test_linear_large_m_slab_counts(M, K):
+    """The 64-wide slab pipeline at its shortest and odd slab counts, partial row blocks and a partial column block:
+    every epilogue against fp64, and the residual read in place or from another buffer."""
+    g = gen(M + K)
+    N = 392
+    x = to_dev(R.bf(torch.randn(M, K, generator=g)), BF)
+    w = to_dev(R.bf(torch.randn(2 * N, K, generator=g) / math.sqrt(K)), BF)
+    ref = x.double() @ w.double().t()
+    # fp32 sums of K products of N(0, 1) / sqrt(K) terms: K eps bounds them with room
+    y32 = ops.linear(x, w[:N].contiguous(), out_dtype=torch.float32)
+    assert torch.allclose(y32.double(), ref[:, :N], rtol=1e-5, atol=1e-5)
+    assert torch.equal(ops.linear(x, w[:N].contiguous()), y32.to(BF))
+    gu = torch.empty(M, 2 * N, dtype=BF, device=DEV)
+    act = ops.linear(x, w, swiglu=True, gu_out=gu)
+    assert torch.equal(gu[:, :N], y32.to(BF))
+    assert torch.equal(act, ops.linear(x, w, swiglu=True))
+    want = R.bf(torch.nn.functional.silu(gu[:, :N].float()).cpu()) * gu[:, N:].float().cpu()
+    assert bf_close(act, want, ulps=4, atol=1e-5)[0]
+    wr = w[:384].contiguous()
+    for dt in (torch.float32, BF):
+        r = to_dev(torch.randn(M, 384, generator=g), dt)
+        out = torch.empty_like(r)
+        ss = ops.linear_residual_big(x, wr, r, out=out)
+        prod = y32[:, :384].to(BF)
+        new = r + prod if dt == torch.float32 else (prod.float() + r.float()).to(BF)
+        assert torch.equal(out, new)
+        blocks = new.double().view(M, 6, 64).pow(2).sum(-1)
+        assert torch.allclose(ss.double(), blocks, rtol=1e-5)
+        assert torch.equal(ops.linear_residual_big(x, wr, r), ss) and torch.equal(r, new)
+
+
+def test_linear_wide_tiles_same_bits():
+    """256 row blocks of 256 fill the chip with 256 x 256 tiles at K >= 1024; a row's bits are those of the 128 x 128
+    tiles that a smaller batch runs."""
+    g = gen(77)
+    M, N, K = 65536 - 37, 248, 1088
+    x = to_dev(R.bf(torch.randn(4133, K, generator=g)), BF)
+    w = to_dev(R.bf(torch.randn(N, K, generator=g) / math.sqrt(K)), BF)
+    rows = torch.arange(M, device=DEV) % 4133
+    big = x[rows]
+    small = ops.linear(x, w)
+    assert torch.equal(ops.linear(big, w), small[rows])
+    small = ops.linear(x, w, out_dtype=torch.float32)
+    assert torch.equal(ops.linear(big, w, out_dtype=torch.float32), small[rows])
+    assert torch.allclose(small.double(), x.double() @ w.double().t(), rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("M,N,K", [(4099, 1536, 512), (8192, 520, 512), (4608, 512, 1536), (5000, 3072, 1024)])
 def test_linear_large_m_tile_shapes_same_bits(M, N, K):
     """Large M: bf16 outputs run 256 x 256 tiles, fp32 outputs at K < 1024 the 256 x 128 tiles; both accumulate

@@ -1,61 +1,67 @@
 // Large-M GEMMs of the prefill / scoring forward: y[M, N] = x[M, K] @ w[N, K]^T, bf16 in, fp32 accumulate.
 //
-// MI355X design (M = tokens or frames x N = 512..4096 x K = 512..2048):
-//   * 256 x 128 output tile per workgroup of 4 wavefronts, each wavefront 128 x 64 (32 fp32 MFMA tiles, 128
-//     accumulator registers), so a wavefront fits in 256 registers and two workgroups share a CU: one
-//     workgroup's barriers, LDS phases and epilogue overlap the other's MFMAs (with 256 x 256 tiles of
-//     128 x 128 per wavefront, one wavefront per SIMD left all of those exposed). Plain products use 256 x 256
-//     tiles of 8 such wavefronts instead (one workgroup per CU, a third fewer global->LDS bytes per flop).
-//   * Operands reach LDS with gfx950's direct global->LDS loads (global_load_lds_dwordx4: lane l of an
-//     instruction lands at LDS base + 16 l), so the prefetch costs no registers; a 3-stage ring of 32-wide K
-//     slices (72 KB) keeps two slices in flight while one feeds the MFMAs. LDS rows are 64 B without padding;
-//     the 16-byte slot of K chunk c in row r is c ^ ((r >> 1) & 3), so the 8 lanes of a fragment-read phase
-//     (8 consecutive rows, one chunk) hit 8 distinct bank groups. A wavefront reads its 12 fragments of a
-//     slice before its 32 MFMAs (pinned with sched_group_barrier).
+// MI355X design (M = tokens or frames x N = 512..4096 x K = 512..3072):
+//   * 128 x 128 output tile per workgroup of 4 wavefronts, each 64 x 64 (16 fp32 MFMA tiles, 64 accumulator
+//     registers), two workgroups per CU: one workgroup's barriers and epilogue overlap the other's MFMAs, and a
+//     packed batch of a few thousand rows still fills the chip.
+//   * What bounds the K loop: with the MFMAs and LDS reads alone it runs at 1820 TFLOP/s (MFMAs alone 2080), with the
+//     loads alone at the rate of the global->LDS stream. That stream is issued as direct loads (buffer_load .. lds,
+//     16 bytes a lane, no registers) of 64-wide K slabs: 8 lanes take a row's whole 128-byte line, 24-29 TB/s over
+//     the chip; 32-wide slabs (64-byte rows) reached 16 TB/s. With real operands the clock then falls with the power
+//     drawn: the loop without an epilogue runs at 1100-1240 TFLOP/s (zero operands: 1490) for every tile shape tried.
+//   * Against 256 x 128 tiles with 32-wide slabs in a three-stage ring (same box, us): N = 512, K = 512 / 1536 + bf16
+//     residual at M = 4099: 18.5 / 35.1 -> 11.2 / 20.4, M = 45057: 46.0 / 92.5 -> 40.7 / 77.7, M = 131136: 122 / 278
+//     -> 111 / 269; SwiGLU N = 1536, K = 512: 20.5 -> 17.8, 154 -> 146, 427 -> 417; Wqkv N = 768: M = 45057 62 -> 53,
+//     M = 131136 153 -> 160 (the one shape that lost).
 //   * Tiles are ordered XCD-aware: workgroup p runs on XCD p % 8, so each XCD gets a contiguous range of
 //     tiles and the N-tiles that share a block of x rows share that XCD's L2.
 //   * The product is formed transposed, C^T = W X^T (the weight fragment is the MFMA A operand), so each
-//     lane ends with 4 consecutive output columns of one row; the epilogue stages each wavefront's quadrant
+//     lane ends with 4 consecutive output columns of one row; the epilogue stages each wavefront's block
 //     through LDS and stores whole rows in 16-byte chunks.
 //   * SwiGLU: the tile's W rows are 64 gate rows and the matching 64 up rows; both land in the same lane,
 //     and the epilogue stores bf16(bf16(silu(bf16(g))) * bf16(u)) over 64 output columns.
-//   * Every row of y is computed by the same code whatever M is (no split of K), so a row's result does not
-//     depend on the other rows of the product.
+//   * Every row of y is computed by the same code whatever M is (no split of K; every tile shape adds the same
+//     32-wide MFMA steps in the same order), so a row's result does not depend on the other rows of the product.
 #include <type_traits>
 
 #include "common.h"
 
 namespace vk {
 
-constexpr int GB_BM = 256;   // rows of x per workgroup
-constexpr int GB_BK = 32;    // K per stage
-constexpr int GB_GM = 8;     // row blocks per group of the tile order
-constexpr int GB_STAGES = 3;
-constexpr int GB_ROWB = GB_BK * 2;                   // bytes per LDS row
-constexpr int GB_XTILEB = GB_BM * GB_ROWB;           // 16 KB
+constexpr int GB_BK = 64;           // K per stage
+constexpr int GB_ROWB = GB_BK * 2;  // bytes per LDS row
 
-// GW wavefronts along the weight rows, each 64 of them; 2 GW wavefronts per workgroup, every one a 128 x 64 block.
-// GW = 2: 256 x 128 tiles, 4 wavefronts, 72 KB of ring (two workgroups per CU); GW = 4: 256 x 256 tiles, 8
-// wavefronts, 96 KB (one workgroup per CU): a third fewer global->LDS bytes per flop.
-template <int GW>
+// A workgroup of RW x GW wavefronts, each 16 FX rows of x by 64 weight rows.
+template <int RW_, int GW_, int FX_>
 struct GbShape {
-  static constexpr int WAVES = 2 * GW;
+  static constexpr int RW = RW_, GW = GW_, FX = FX_;
+  static constexpr int WAVES = RW * GW;
+  static constexpr int WROWS = 16 * FX;                                // rows of x per wavefront
+  static constexpr int BM = RW * WROWS;                                // rows of x per workgroup
   static constexpr int BW = 64 * GW;                                   // rows of w per workgroup
-  static constexpr int WTILEB = BW * GB_ROWB;                          // 8 / 16 KB
-  static constexpr int STAGEB = GB_XTILEB + WTILEB;                    // 24 / 32 KB
-  static constexpr size_t SMEM = static_cast<size_t>(GB_STAGES) * STAGEB;  // 72 / 96 KB
-  static constexpr int XLOADS = 16 / WAVES;                            // x instructions per wave per stage
-  static constexpr int LOADS = XLOADS + 2;                             // + 2 w instructions
-  static constexpr int WG_PER_CU = GW == 2 ? 2 : 1;
+  static constexpr int XTILEB = BM * GB_ROWB, WTILEB = BW * GB_ROWB;
+  static constexpr int STAGEB = XTILEB + WTILEB;
+  static constexpr size_t SMEM = 2 * static_cast<size_t>(STAGEB);
+  static constexpr int RPL = 1024 / GB_ROWB;                           // rows per direct-load instruction
+  static constexpr int XLOADS = BM / RPL / WAVES;                      // x instructions per wave per stage
+  static constexpr int WLOADS = BW / RPL / WAVES;
+  static constexpr int LOADS = XLOADS + WLOADS;
+  static constexpr int WG_PER_CU = SMEM > 81920 ? 1 : 2;
+  static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
 };
+using GbWide = GbShape<2, 4, 8>;    // 256 x 256, 128 KB: one workgroup of 8 wavefronts per CU
+using GbSquare = GbShape<2, 2, 4>;  // 128 x 128, 64 KB: two workgroups per CU
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// One 16-byte direct global->LDS load per lane (lane l lands at dst + 16 l). A plain device function: written in
-// a kernel template with arguments that depend on its parameters, the builtin makes the host pass drop the
-// kernel's launch stub.
-__device__ __forceinline__ void gb_load_lds(const bf16_t *src, char *dst) {
-  __builtin_amdgcn_global_load_lds(src, (lds_void *)dst, 16, 0, 0);
+// A buffer descriptor over `bytes` bytes from p (raw, unstrided), and one 16-byte direct buffer->LDS load per lane:
+// lane l reads p + vo + so (zero past the end) into dst + 16 l. Plain device functions: written in a kernel template
+// with arguments that depend on its parameters, the builtin makes the host pass drop the kernel's launch stub.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gb_rsrc(const bf16_t *p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p), 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ void gb_buf_lds(__amdgpu_buffer_rsrc_t r, char *dst, uint32_t vo, uint32_t so) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)dst, 16, vo, so, 0, 0);
 }
 
 // s_waitcnt immediate that waits for vmcnt <= n and leaves expcnt / lgkmcnt unconstrained (gfx9 encoding:
@@ -108,13 +114,12 @@ struct GbQkv {
   const void *resid_in;  // the old residual rows [M, N] (NULL: the output itself, updated in place)
 };
 
-template <int EPI, int GW>
-__global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
+template <int EPI, class SH>
+__global__ __launch_bounds__(64 * SH::WAVES, SH::WAVES_PER_SIMD) void gemm_big_kernel(
     const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, void *__restrict__ y, int64_t M, int N, int K,
-    int tiles_n, int tiles_total, const GbQkv qa) {
-  using SH = GbShape<GW>;
-  constexpr int GB_STAGEB = SH::STAGEB, GB_LOADS = SH::LOADS, NWAVES = SH::WAVES;
-  constexpr size_t GB_SMEM = SH::SMEM;
+    int tiles_n, int tiles_total, int group_m, const GbQkv qa) {
+  constexpr int GB_STAGEB = SH::STAGEB, GB_LOADS = SH::LOADS, NWAVES = SH::WAVES, GW = SH::GW, FX = SH::FX;
+  constexpr int GB_BM = SH::BM, GB_XTILEB = SH::XTILEB, WROWS = SH::WROWS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr bool SWIGLU = EPI == GB_SWIGLU, OUT_F32 = EPI == GB_F32, RESID = EPI == GB_RESID;
   constexpr bool RESID32 = EPI == GB_RESID_F32;
@@ -131,248 +136,248 @@ __global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
   const int xcd = p & 7, idx = p >> 3;
   const int q8 = tiles_total >> 3, r8 = tiles_total & 7;
   const int tile = xcd * q8 + min(xcd, r8) + idx;
-  // logical order: groups of GB_GM row blocks, each walked column block by column block (GB_GM row blocks
-  // per column block), so an XCD's resident workgroups share GB_GM A blocks and a few weight blocks in its
+  // logical order: groups of group_m row blocks, each walked column block by column block (group_m row blocks
+  // per column block), so an XCD's resident workgroups share group_m A blocks and a few weight blocks in its
   // L2 instead of every weight block (a bijection: the last group has the remaining row blocks)
   const int tiles_m = tiles_total / tiles_n;
-  const int grp = tile / (GB_GM * tiles_n), first_m = grp * GB_GM;
-  const int gm = min(tiles_m - first_m, GB_GM), in_grp = tile - grp * GB_GM * tiles_n;
+  const int grp = tile / (group_m * tiles_n), first_m = grp * group_m;
+  const int gm = min(tiles_m - first_m, group_m), in_grp = tile - grp * group_m * tiles_n;
   const int mt = first_m + in_grp % gm, nt = in_grp / gm;
   const int64_t m0 = static_cast<int64_t>(mt) * GB_BM;
   const int n0 = nt * OUT_COLS;
 
-  // direct-load sources: instruction q of an operand tile covers its rows 16 q .. 16 q + 15 (x: q < 16,
-  // w: q < 4 GW); wave w issues q = w + NWAVES i. Lane l -> row 16 q + l / 4, LDS slot l % 4, K chunk slot ^ swizzle.
-  const bf16_t *xsrc[SH::XLOADS];
-  const bf16_t *wsrc[2];
-#pragma unroll
-  for (int i = 0; i < SH::XLOADS; ++i) {
-    const int r = 16 * (wid + NWAVES * i) + (lane >> 2);
-    const int c = (lane & 3) ^ ((r >> 1) & 3);
-    int64_t gr = m0 + r;
-    gr = gr < M ? gr : M - 1;
-    xsrc[i] = x + gr * K + 8 * c;
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = 16 * (wid + NWAVES * i) + (lane >> 2);
-    const int c = (lane & 3) ^ ((r >> 1) & 3);
-    int wr;
-    if (SWIGLU) {  // tile rows 0..32 GW - 1: gate rows n0.., the next 32 GW: the matching up rows N + n0..
-      int colr = n0 + (r & (32 * GW - 1));
-      colr = colr < N ? colr : N - 1;
-      wr = colr + (r >= 32 * GW ? N : 0);
-    } else {
-      wr = n0 + r;
-      wr = wr < N ? wr : N - 1;
-    }
-    wsrc[i] = w + static_cast<int64_t>(wr) * K + 8 * c;
-  }
-  auto issue = [&](int stage, int k0) {
-    char *base = smem + (stage % GB_STAGES) * GB_STAGEB;
-#pragma unroll
-    for (int i = 0; i < SH::XLOADS; ++i) gb_load_lds(xsrc[i] + k0, base + (wid + NWAVES * i) * 1024);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) gb_load_lds(wsrc[i] + k0, base + GB_XTILEB + (wid + NWAVES * i) * 1024);
-  };
-
-  f32x4 acc[4][8];
+  f32x4 acc[4][FX];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < FX; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int fr = lane & 15, fg = lane >> 4;
-  // fragment byte offsets inside a tile: row R, chunk fg -> R * 64 + 16 * (fg ^ ((R >> 1) & 3))
-  int xoff[8], woff[4];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int R = wm * 128 + 16 * j + fr;
-    xoff[j] = R * GB_ROWB + 16 * (fg ^ ((R >> 1) & 3));
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int R = SWIGLU ? ((i < 2 ? 0 : 32 * GW) + wn * 32 + 16 * (i & 1) + fr) : (wn * 64 + 16 * i + fr);
-    woff[i] = GB_XTILEB + R * GB_ROWB + 16 * (fg ^ ((R >> 1) & 3));
-  }
-
-  // The plain, fp32 and SwiGLU epilogues (whose values live across the loop leave room for a second set of
-  // fragment registers) run a software-pipelined K loop: a wavefront reads its 12 fragments of slice kt + 1
-  // while its 32 MFMAs of slice kt run, from two register sets (the loop unrolled by two). Slice kt + 1 must
-  // then be whole in LDS one slice earlier, and slice kt + 3 goes into slice kt's slot once every wavefront has
-  // its fragments of slice kt in registers, so two slices stay in flight during the MFMAs, as with reads right
-  // before them. The other epilogues would spill with the second set; they read a slice's fragments right
-  // before its MFMAs.
-  constexpr bool PIPE = EPI == GB_BF16 || EPI == GB_F32 || EPI == GB_SWIGLU;
-  const int nk = K / GB_BK;
-#pragma unroll
-  for (int s = 0; s < GB_STAGES - 1; ++s)
-    if (s < nk) issue(s, s * GB_BK);
-  auto read_frags = [&](int kt, bf16x8(&xf)[8], bf16x8(&wf)[4]) {
-    const char *base = smem + (kt % GB_STAGES) * GB_STAGEB;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) xf[j] = *reinterpret_cast<const bf16x8 *>(base + xoff[j]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) wf[i] = *reinterpret_cast<const bf16x8 *>(base + woff[i]);
-  };
-  auto mfmas = [&](const bf16x8(&xf)[8], const bf16x8(&wf)[4]) {
+  auto mfmas = [&](const bf16x8(&xf)[FX], const bf16x8(&wf)[4]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < FX; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
   };
-  if constexpr (PIPE) {
-    // this thread's loads of slice kt + 1 are done once at most slice kt + 2's remain, and its fragment reads
-    // of slice kt are done; after the barrier slice kt + 1 is whole in LDS and slice kt's slot is free for
-    // kt + 3. A bare s_barrier: __syncthreads() would add a release fence that drains every outstanding load,
-    // the prefetched slices included.
-    auto next_slice = [&](int kt) {
+  // one LDS read of the next slice between the MFMAs of this one, then the MFMAs left over
+#define GB_INTERLEAVE()                                                        \
+  do {                                                                         \
+    constexpr int per_ = 4 * FX / (FX + 4);                                    \
+    _Pragma("unroll") for (int r_ = 0; r_ < FX + 4; ++r_) {                    \
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                       \
+      __builtin_amdgcn_sched_group_barrier(0x008, per_, 0);                    \
+    }                                                                          \
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * FX - per_ * (FX + 4), 0);  \
+  } while (0)
+  // Two stages of 64-wide K slabs (LDS rows of 128 bytes: a direct load's 8 lanes of a row take one whole
+  // cache line; with 64-byte rows the same stream ran at 16 instead of 24 TB/s). The stage holds a slab's
+  // two 32-wide slices; a wavefront reads the next slice's fragments while this one's MFMAs run, from two
+  // register sets. Once every wavefront has its fragments of slab kt in registers (the barrier), slab kt + 2
+  // goes into its stage; slab kt + 1 had the time of a whole slab to land. Buffer loads: rows past M or N are
+  // past the descriptor's end and read as zero (they only reach outputs that are not stored), and the K offset
+  // and row block ride in the scalar offset, so a source takes one register.
+  // LDS slot of K chunk c (16 bytes) in row r: c ^ ((r >> 1) & 7), so 16 consecutive rows of a chunk cover all
+  // 64 banks.
+  const int64_t xrows = M - m0 < GB_BM ? M - m0 : GB_BM;
+  const auto xr = gb_rsrc(x + m0 * K, static_cast<uint32_t>(xrows) * K * 2);
+  constexpr int HALVES = SWIGLU ? 2 : 1;  // SwiGLU: gate rows n0.. of w, then the matching up rows N + n0..
+  const uint32_t wrows = N - n0 < SH::BW / HALVES ? N - n0 : SH::BW / HALVES;
+  const auto wr = gb_rsrc(w + static_cast<int64_t>(n0) * K, wrows * K * 2);
+  const auto wr2 = gb_rsrc(w + static_cast<int64_t>(SWIGLU ? N + n0 : n0) * K, wrows * K * 2);
+  const int lr = SH::RPL * wid + (lane >> 3);
+  const uint32_t vo = static_cast<uint32_t>(lr) * K * 2 + 16 * ((lane & 7) ^ ((lr >> 1) & 7));
+  const uint32_t rstep = SH::RPL * NWAVES * static_cast<uint32_t>(K) * 2;
+  auto issue = [&](int stage, int kt) {
+    char *base = smem + stage * GB_STAGEB;
+    const uint32_t so = static_cast<uint32_t>(kt) * 128;
+#pragma unroll
+    for (int i = 0; i < SH::XLOADS; ++i) gb_buf_lds(xr, base + (wid + NWAVES * i) * 1024, vo, so + i * rstep);
+#pragma unroll
+    for (int i = 0; i < SH::WLOADS; ++i) {
+      constexpr int HL = SH::WLOADS / HALVES;
+      const int ih = i >= HL ? i - HL : i;
+      gb_buf_lds(i >= HL ? wr2 : wr, base + GB_XTILEB + (wid + NWAVES * i) * 1024, vo, so + ih * rstep);
+    }
+  };
+  const int sw = 16 * (fg ^ ((fr >> 1) & 7));
+  const int xo = (wm * WROWS + fr) * 128 + sw;
+  int wo[2];  // fragments 0, 1 and 2, 3 (SwiGLU: gate and up rows)
+  wo[0] = GB_XTILEB + ((SWIGLU ? wn * 32 : wn * 64) + fr) * 128 + sw;
+  wo[1] = SWIGLU ? wo[0] + 32 * GW * 128 : wo[0] + 32 * 128;
+  auto read_frags = [&](int stage, int kk, bf16x8(&xf)[FX], bf16x8(&wf)[4]) {
+    const char *base = smem + stage * GB_STAGEB;
+#pragma unroll
+    for (int j = 0; j < FX; ++j) xf[j] = *reinterpret_cast<const bf16x8 *>(base + (xo ^ (64 * kk)) + j * 2048);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      wf[i] = *reinterpret_cast<const bf16x8 *>(base + (wo[i >> 1] ^ (64 * kk)) + (i & 1) * 2048);
+  };
+  const int nk = K / 64;
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  const int first = nk & 1;  // slab 0's stage
+  issue(first, 0);
+  if (nk > 1) {
+    issue(first ^ 1, 1);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(GB_LOADS));
+  } else {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  }
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  bf16x8 xa[FX], wa[4], xb[FX], wb[4];
+  if (FX == 4) read_frags(first, 0, xa, wa);
+  // The residual epilogues' operands (old rows, bias) are loaded in the last slab but one, behind the last direct loads,
+  // so their round trips pass under its MFMAs (M = 131136, N = 512: 115 -> 111 us at K = 512, 290 -> 269 at K = 1536).
+  // The QKV epilogues' (QK-norm weights, every row's rotary position; the table rows, which depend on the positions,
+  // go one row group ahead) measured the same there or after the loop, and are loaded after it.
+  u32x2 res_old[RESID ? FX : 1][4];
+  f32x4 r32_old[RESID32 ? FX : 1][4];
+  f32x4 res_b4[(RESID || RESID32) ? 4 : 1];
+  using NwT = typename std::conditional<W32, f32x4, u32x2>::type;
+  NwT qk_nw[QKV ? 4 : 1];
+  int qk_rp[QKV ? FX : 1];
+  const int qk_hd = (n0 + wn * 64) >> 6;  // GB_QKV: this wavefront's head (64 columns, wave-uniform)
+  const bool qk_rot = QKV && qk_hd < qa.H + qa.HKV;
+  const void *qk_w = QKV ? (qk_hd < qa.H ? qa.qw : qa.kw) : nullptr;
+  auto prefetch = [&]() {
+    if constexpr (RESID || RESID32) {
+#pragma unroll
+      for (int j = 0; j < FX; ++j) {
+        int64_t rrow = m0 + wm * WROWS + 16 * j + fr;
+        rrow = rrow < M ? rrow : M - 1;
+        const void *old = qa.resid_in ? qa.resid_in : y;
+        const int64_t at = rrow * N + n0 + wn * 64 + 4 * fg;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (RESID)
+            res_old[j][i] = *reinterpret_cast<const u32x2 *>(static_cast<const bf16_t *>(old) + at + 16 * i);
+          else
+            r32_old[j][i] = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(old) + at + 16 * i);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        res_b4[i] = qa.bias != nullptr ? *reinterpret_cast<const f32x4 *>(qa.bias + n0 + wn * 64 + 16 * i + 4 * fg)
+                                       : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  auto load_qkv = [&]() {
+    if constexpr (QKV) {
+      if (qk_w != nullptr) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (W32)
+            qk_nw[i] = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(qk_w) + 16 * i + 4 * fg);
+          else
+            qk_nw[i] = *reinterpret_cast<const u32x2 *>(static_cast<const bf16_t *>(qk_w) + 16 * i + 4 * fg);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < FX; ++j) {
+        int64_t rrow = m0 + wm * WROWS + 16 * j + fr;
+        rrow = rrow < M ? rrow : M - 1;
+        int64_t rp = qa.rope_pos != nullptr ? qa.rope_pos[rrow] : qa.pos[rrow];
+        qk_rp[j] = static_cast<int>(rp < 0 ? 0 : (rp >= qa.table_rows ? qa.table_rows - 1 : rp));
+      }
+    }
+  };
+
+  // Slab kt: its second slice's fragments are read under its first slice's MFMAs; once every wavefront has them in
+  // registers and slab kt + 1 is whole in LDS (the waits and the barrier), slab kt + 2 is issued into this stage and
+  // the next slab's first fragments are read under the second slice's MFMAs. A bare s_barrier: __syncthreads()
+  // would also wait for the epilogue's operands, which go out in the last slab but one.
+  auto landed = [&](bool loads) {
+    if (loads) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // (the stage is a compile-time parity: its LDS offsets are then immediates; with a run-time stage the loop ran 3-15%
+  // slower)
+  auto slab = [&](auto stage, int kt) {
+    read_frags(stage, 1, xb, wb);
+    mfmas(xa, wa);
+    GB_INTERLEAVE();
+    landed(true);
+    issue(stage, kt + 2);
+    read_frags(stage ^ 1, 0, xa, wa);
+    mfmas(xb, wb);
+    GB_INTERLEAVE();
+  };
+  auto last_but_one = [&](auto stage) {
+    read_frags(stage, 1, xb, wb);
+    mfmas(xa, wa);
+    GB_INTERLEAVE();
+    landed(true);
+    prefetch();
+    read_frags(stage ^ 1, 0, xa, wa);
+    mfmas(xb, wb);
+    GB_INTERLEAVE();
+  };
+  auto last = [&](auto stage) {
+    read_frags(stage, 1, xb, wb);
+    mfmas(xa, wa);
+    GB_INTERLEAVE();
+    landed(false);  // every wavefront has finished reading the ring: the epilogue stages through it
+    mfmas(xb, wb);
+  };
+  if constexpr (FX == 8) {
+    // no registers for a second set of fragments beside 128 accumulators: a slab's 24 fragments are read, its stage is
+    // refilled once every wavefront has them, and the next slab is waited for after the MFMAs
+    auto step = [&](auto stage, int kt) {
+      read_frags(stage, 0, xa, wa);
+      read_frags(stage, 1, xb, wb);
+      mfmas(xa, wa);
+      landed(false);
+      if (kt + 2 < nk) issue(stage, kt + 2);
+      mfmas(xb, wb);
       if (kt + 2 < nk)
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(GB_LOADS));
       else
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (kt + GB_STAGES < nk) issue(kt + GB_STAGES, (kt + GB_STAGES) * GB_BK);
     };
-    // one LDS read of the next slice between every two MFMAs of this one, then the last 8 MFMAs
-#define GB_INTERLEAVE()                                  \
-  do {                                                   \
-    _Pragma("unroll") for (int r_ = 0; r_ < 12; ++r_) {  \
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); \
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0); \
-    }                                                    \
-    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);   \
-  } while (0)
-    bf16x8 xa[8], wa[4], xb[8], wb[4];
-    // slice 0 whole in LDS (slice 2 then goes into the ring's third slot), its fragments read
-    if (nk > 1)
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(GB_LOADS));
-    else
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (GB_STAGES - 1 < nk) issue(GB_STAGES - 1, (GB_STAGES - 1) * GB_BK);
-    read_frags(0, xa, wa);
-    // Pairs of slices; the second step of the last pair may have no next slice: it then re-reads slice nk - 1
-    // (its LDS slot is no longer written), so no branch separates a step's reads from its MFMAs and the
-    // scheduler can interleave them. An odd count leaves slice nk - 1 in xa for the step after the loop.
-    // next_slice(j) with j + 1 == nk waits for every load and passes a barrier; it issues nothing.
     int kt = 0;
-    for (; kt + 1 < nk; kt += 2) {
-      next_slice(kt);
-      read_frags(kt + 1, xb, wb);
-      mfmas(xa, wa);
-      GB_INTERLEAVE();
-      next_slice(kt + 1);  // (past the last slice: only the waits and the barrier)
-      read_frags(min(kt + 2, nk - 1), xa, wa);
-      mfmas(xb, wb);
-      GB_INTERLEAVE();
+    if (nk & 1) step(odd, kt++);
+    for (; kt < nk; kt += 2) {
+      step(even, kt);
+      step(odd, kt + 1);
     }
-    if (kt < nk) {
-      __builtin_amdgcn_s_waitcnt(0xC07F);
-      mfmas(xa, wa);
-    }
-#undef GB_INTERLEAVE
+    prefetch();
   } else {
-    for (int kt = 0; kt < nk; ++kt) {
-      // this thread's loads of stage kt are done once at most (stages issued after it) x GB_LOADS remain
-      if (kt + 1 < nk)
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(GB_LOADS));
-      else
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-      // Every thread's slice of stage kt has landed (the wait above), so after the barrier the whole stage is
-      // in LDS and stage kt - 1's slot is free. A bare s_barrier: __syncthreads() would add a release fence
-      // that drains every outstanding load, the prefetched stage included.
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      if (kt + GB_STAGES - 1 < nk) issue(kt + GB_STAGES - 1, (kt + GB_STAGES - 1) * GB_BK);
-      bf16x8 xf[8], wf[4];
-      read_frags(kt, xf, wf);
-      mfmas(xf, wf);
-      // keep that order: the scheduler would otherwise sink each W read next to its 8 MFMAs
-      __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);  // 12 LDS reads
-      __builtin_amdgcn_sched_group_barrier(0x008, 32, 0);  // then the 32 MFMAs
+    // the last slab is always in stage 1, so an odd count has a step of its own in front
+    int kt = 0;
+    if (nk & 1) {
+      if (nk > 1) slab(odd, kt++);
     }
+    for (; kt + 3 < nk; kt += 2) {
+      slab(even, kt);
+      slab(odd, kt + 1);
+    }
+    if (nk > 1)
+      last_but_one(even);
+    else
+      prefetch();
+    last(odd);
   }
+#undef GB_INTERLEAVE
 
   // Epilogue through LDS: a lane holds 4 consecutive columns of one row per (i, j), so direct stores would
-  // write 16 rows x 16-32 B per instruction. Each wavefront instead stages its 128-row quadrant in its own
+  // write 16 rows x 16-32 B per instruction. Each wavefront instead stages its block of rows in its own
   // quarter of the (now idle) ring, a pass of rows at a time (row pitch + 16 B against bank conflicts), and
   // stores 16-byte chunks whose lanes cover whole rows.
-  // The epilogue's global operands are loaded here, before the barrier, so their round trips overlap the other
-  // wavefronts' last MFMAs instead of being taken one 16-row group at a time: the residual rows and the bias
-  // (GB_RESID), the QK-norm weights and every row's rotary position (GB_QKV; the table rows, which depend on the
-  // positions, go one group ahead inside the loop).
-  const int fr_e = lane & 15, fg_e = lane >> 4;
-  u32x2 res_old[RESID ? 8 : 1][4];
-  f32x4 res_b4[(RESID || RESID32) ? 4 : 1];
-  // GB_RESID_F32: the old fp32 residual of two 16-row groups (the current one and the next, loaded one group ahead;
-  // all 8 would take 128 registers beside the accumulators)
-  f32x4 r32_old[RESID32 ? 2 : 1][4];
-  auto r32_load = [&](int j, f32x4 (&dst)[4]) {
-    int64_t rrow = m0 + wm * 128 + 16 * j + fr_e;
-    rrow = rrow < M ? rrow : M - 1;
-    const float *yrow = static_cast<const float *>(qa.resid_in ? qa.resid_in : y) + rrow * N + n0 + wn * 64;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = *reinterpret_cast<const f32x4 *>(yrow + 16 * i + 4 * fg_e);
-  };
-  using NwT = typename std::conditional<W32, f32x4, u32x2>::type;
-  NwT qk_nw[QKV ? 4 : 1];
-  int qk_rp[QKV ? 8 : 1];
-  const int qk_hd = (n0 + wn * 64) >> 6;  // GB_QKV: this wavefront's head (64 columns, wave-uniform)
-  const bool qk_rot = QKV && qk_hd < qa.H + qa.HKV;
-  const void *qk_w = QKV ? (qk_hd < qa.H ? qa.qw : qa.kw) : nullptr;
-  if (RESID32) {
-    r32_load(0, r32_old[0]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      res_b4[i] = qa.bias != nullptr ? *reinterpret_cast<const f32x4 *>(qa.bias + n0 + wn * 64 + 16 * i + 4 * fg_e)
-                                     : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  if (RESID) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      int64_t rrow = m0 + wm * 128 + 16 * j + fr_e;
-      rrow = rrow < M ? rrow : M - 1;
-      const bf16_t *yrow = static_cast<const bf16_t *>(qa.resid_in ? qa.resid_in : y) + rrow * N + n0 + wn * 64;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) res_old[j][i] = *reinterpret_cast<const u32x2 *>(yrow + 16 * i + 4 * fg_e);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      res_b4[i] = qa.bias != nullptr ? *reinterpret_cast<const f32x4 *>(qa.bias + n0 + wn * 64 + 16 * i + 4 * fg_e)
-                                     : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  if (qk_rot) {
-    if (qk_w != nullptr) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (W32)
-          qk_nw[i] = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(qk_w) + 16 * i + 4 * fg_e);
-        else
-          qk_nw[i] = *reinterpret_cast<const u32x2 *>(static_cast<const bf16_t *>(qk_w) + 16 * i + 4 * fg_e);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      int64_t rrow = m0 + wm * 128 + 16 * j + fr_e;
-      rrow = rrow < M ? rrow : M - 1;
-      int64_t rp = qa.rope_pos != nullptr ? qa.rope_pos[rrow] : qa.pos[rrow];
-      qk_rp[j] = static_cast<int>(rp < 0 ? 0 : (rp >= qa.table_rows ? qa.table_rows - 1 : rp));
-    }
-  }
   // GB_QKV: the rotary table entries of 16-row group j (lane: its row's 4 consecutive entries at 16 i + 4 fg,
   // i = 0, 1): four fp32 values (GB_QKV) or four bf16 values in two words (GB_QKV_BF16) per table and i
   using TabT = typename std::conditional<TAB_F32, f32x4, u32x2>::type;
   auto qk_tables = [&](int j, TabT (&c)[2], TabT (&sn)[2]) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int64_t ti = static_cast<int64_t>(qk_rp[j]) * 32 + 16 * i + 4 * fg_e;
+      const int64_t ti = static_cast<int64_t>(qk_rp[j]) * 32 + 16 * i + 4 * fg;
       if constexpr (TAB_F32) {
         c[i] = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(qa.cos_t) + ti);
         sn[i] = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(qa.sin_t) + ti);
@@ -383,22 +388,24 @@ __global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
     }
   };
   TabT qk_c[2][2], qk_s[2][2];  // two row groups' table entries: the current one and the next
-  if (qk_rot) qk_tables(0, qk_c[0], qk_s[0]);
-  __syncthreads();  // every wavefront has finished reading the ring
+  if (qk_rot) {
+    load_qkv();
+    qk_tables(0, qk_c[0], qk_s[0]);
+  }
   constexpr int ESZ = (OUT_F32 || RESID32) ? 4 : 2;   // output element bytes
   constexpr int QCOLS = SWIGLU ? 32 : 64;             // output columns of a wavefront
   constexpr int RB = QCOLS * ESZ;                     // bytes of one quadrant row
   constexpr int PITCH = RB + 16;
   // rows staged per pass: what fits this wavefront's share of the ring (a power of two, 32..128)
-  constexpr int STG_BYTES = static_cast<int>(GB_SMEM / NWAVES);
-  constexpr int PASS_ROWS = 128 * PITCH <= STG_BYTES ? 128 : (64 * PITCH <= STG_BYTES ? 64 : 32);
+  constexpr int STG_BYTES = static_cast<int>(SH::SMEM / NWAVES);
+  constexpr int PASS_ROWS = WROWS * PITCH <= STG_BYTES ? WROWS : (WROWS > 64 && 64 * PITCH <= STG_BYTES ? 64 : 32);
   constexpr int CPR = RB / 16;                        // 16-byte chunks per row
   static_assert(PASS_ROWS * PITCH <= STG_BYTES, "epilogue staging exceeds the wavefront's share of LDS");
   char *stg = smem + wid * STG_BYTES;
-  const int64_t qrow0 = m0 + wm * 128;
+  const int64_t qrow0 = m0 + wm * WROWS;
   const int qcol0 = n0 + wn * QCOLS;
 #pragma unroll
-  for (int pass = 0; pass < 128 / PASS_ROWS; ++pass) {
+  for (int pass = 0; pass < WROWS / PASS_ROWS; ++pass) {
 #pragma unroll
     for (int jj = 0; jj < PASS_ROWS / 16; ++jj) {
       const int j = pass * (PASS_ROWS / 16) + jj;
@@ -427,13 +434,12 @@ __global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
         ss += __shfl_xor(ss, 32, 64);
         if (live && fg == 0) qa.ss_out[rrow * (N >> 6) + (qcol0 >> 6)] = ss;
       } else if (RESID32) {
-        // lane: row 16 j + fr, columns qcol0 + 16 i + 4 fg + e (the same elements r32_load read for it)
-        if (j + 1 < 8) r32_load(j + 1, r32_old[(j + 1) & 1]);
+        // lane: row 16 j + fr, columns qcol0 + 16 i + 4 fg + e (the same elements prefetch read for it)
         const int64_t rrow = qrow0 + 16 * j + fr;
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const f32x4 old = r32_old[j & 1][i];
+          const f32x4 old = r32_old[j][i];
           const f32x4 b4 = res_b4[i];
           f32x4 o;
 #pragma unroll
@@ -464,7 +470,7 @@ __global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
         }
         if (hd < qa.H + qa.HKV) {  // q or k head: QK-norm, then the rotation
           // the next group's table entries go out before this group's arithmetic
-          if (j + 1 < 8) qk_tables(j + 1, qk_c[(j + 1) & 1], qk_s[(j + 1) & 1]);
+          if (j + 1 < FX) qk_tables(j + 1, qk_c[(j + 1) & 1], qk_s[(j + 1) & 1]);
           if (qk_w != nullptr) {
             float ss = 0.f;
 #pragma unroll
@@ -552,7 +558,7 @@ __global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
         }
       }
     }
-    // GB_QKV with a cache: the cache row and position of the quadrant's 128 rows, one pair of rows per lane (rows
+    // GB_QKV with a cache: the cache row and position of the pass's (up to 128) rows, one pair of rows per lane (rows
     // lane and 64 + lane), handed to the lane that stores a row's chunk by a lane shuffle below
     int cs_lo = 0, cs_hi = 0, cp_lo = 0, cp_hi = 0;
     if (QKV && (qcol0 >> 6) >= qa.H && qa.kc != nullptr) {
@@ -600,31 +606,39 @@ __global__ __launch_bounds__(128 * GW, 4 / GW) void gemm_big_kernel(
   }
 }
 
-template <int EPI, int GW>
-static int launch_big_gw(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int N, int K, const GbQkv &qa,
-                         hipStream_t s) {
-  using SH = GbShape<GW>;
-  VK_RAISE_LDS_ONCE((gemm_big_kernel<EPI, GW>), SH::SMEM, "linear");
-  constexpr int OUT_COLS = EPI == GB_SWIGLU ? 32 * GW : 64 * GW;
+template <int EPI, class SH>
+static int launch_big_shape(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int N, int K, const GbQkv &qa,
+                            hipStream_t s) {
+  VK_RAISE_LDS_ONCE((gemm_big_kernel<EPI, SH>), SH::SMEM, "linear");
+  constexpr int OUT_COLS = EPI == GB_SWIGLU ? SH::BW / 2 : SH::BW;
   const int tiles_n = (N + OUT_COLS - 1) / OUT_COLS;
-  const int64_t tiles_m = (M + GB_BM - 1) / GB_BM;
+  const int64_t tiles_m = (M + SH::BM - 1) / SH::BM;
   const int64_t total = tiles_m * tiles_n;
   if (total >= (int64_t(1) << 31)) return fail(VK_ERR_ARG, "linear: too many tiles");
-  gemm_big_kernel<EPI, GW><<<static_cast<unsigned>(total), 128 * GW, SH::SMEM, s>>>(x, w, y, M, N, K, tiles_n,
-                                                                                    static_cast<int>(total), qa);
+  // (the descriptors hold a row block's bytes in 32 bits)
+  if (K > (1 << 22)) return fail(VK_ERR_ARG, "linear: K %d too large", K);
+  // Row blocks per group of the tile order: an XCD has 64 workgroups resident, 16 x 4 tiles for few column blocks
+  // (M = 131136, N = 512, K = 1536: 230 -> 198 us for the loop alone against groups of 8); while an XCD's share is
+  // below a few such groups, 8 (M = 9000, N = 512, K = 3072: 48 -> 41 us against 16).
+  const int group_m = tiles_n <= 4 && total >= 2048 ? 16 : 8;
+  gemm_big_kernel<EPI, SH><<<static_cast<unsigned>(total), 64 * SH::WAVES, SH::SMEM, s>>>(
+      x, w, y, M, N, K, tiles_n, static_cast<int>(total), group_m, qa);
   return VK_OK;
 }
 
-// 256 x 256 tiles where they measured faster (same bits either way, M = 131136 and 4096): bf16 outputs at every K
-// (K 512 / 1536 / 2048: 8 / 4 / 10% faster) and fp32 outputs from K = 1024 (3 / 10% at 1536 / 2048, 1.5% slower at
-// 512). The SwiGLU, residual and Wqkv epilogues run 2-8% slower on them: with one workgroup per CU their epilogue
-// no longer overlaps another workgroup's K loop.
 template <int EPI>
 static int launch_big(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int N, int K, const GbQkv &qa,
                       hipStream_t s) {
-  const bool wide = EPI == GB_BF16 || (EPI == GB_F32 && K >= 1024);
-  if (wide) return launch_big_gw<EPI, 4>(x, w, y, M, N, K, qa, s);
-  return launch_big_gw<EPI, 2>(x, w, y, M, N, K, qa, s);
+  // 256 x 256 tiles read a third fewer bytes into LDS per flop, but their epilogue runs alone on its CU: the faster
+  // ones only for the plain epilogues at a long K, and only where they fill the resident rounds (one workgroup per
+  // CU). N = 512, K = 3072: M = 32000 (250 tiles) 97 -> 84 us, 131136 (1026) 474 -> 442, but 45057 (354) 154 -> 160,
+  // 16000 (126) 49 -> 73; N = 512 or 1536, K = 512: 2-30% slower at every M.
+  if constexpr (EPI == GB_BF16 || EPI == GB_F32) {
+    const int64_t tiles = (M + GbWide::BM - 1) / GbWide::BM * ((N + GbWide::BW - 1) / GbWide::BW);
+    const int64_t cus = device_cus_cached(), rounds = (tiles + cus - 1) / cus;
+    if (K >= 1024 && 8 * tiles >= 7 * rounds * cus) return launch_big_shape<EPI, GbWide>(x, w, y, M, N, K, qa, s);
+  }
+  return launch_big_shape<EPI, GbSquare>(x, w, y, M, N, K, qa, s);
 }
 
 // Entry used by vk_linear for large M and by vk_gemm_rows (K % 64 == 0: an even number of K slices; N % 8 == 0:
