@@ -380,6 +380,21 @@ int vk_attention_backward_prefixed(const void *q, const void *k, const void *v, 
                                    float *dv, int32_t H, int32_t HKV, int32_t D, void *stream);
 
 /*
+ * vk_attention_backward with the query rows of long key blocks split over several work items. k_plan holds n_kblocks
+ * entries (sequence, first key of a 128-key block, first row, -rows, slot): the block's gradients from `rows` of the
+ * sequence's query rows from its row `first row` (>= the first key); slot < 0 writes dk / dv (a block that is one
+ * entry), slot >= 0 the partial block `slot` of part_k / part_v ([slots, 128, HKV, D] fp32, a caller's workspace, no
+ * initial value). red holds n_red entries (first packed row, keys, first slot, slots): the split blocks, whose partial
+ * blocks are summed in slot order into dk / dv. No reference counterpart of its own (the same sums, regrouped).
+ */
+int vk_attention_backward_chunked(const void *q, const void *k, const void *v, const void *out, const void *dout,
+                                  const float *lse, const int32_t *cu, int32_t n_seq, const int32_t *q_plan,
+                                  int32_t n_qblocks, const int32_t *k_plan, int32_t n_kblocks, int64_t n_rows,
+                                  int64_t stride_tok, const int32_t *red, int32_t n_red, float *part_k, float *part_v,
+                                  float *dd, float *dq, float *dk, float *dv, int32_t H, int32_t HKV, int32_t D,
+                                  void *stream);
+
+/*
  * Weight gradient of a linear layer over packed rows: out[Ka, Kb] = a^T b = sum_r a[r, ka] b[r, kb] for a [N, Ka]
  * (the layer's output gradient) and b [N, Kb] (its input), bf16 row-major with row strides lda / ldb (elements,
  * multiples of 8); fp32 accumulation, the N rows split into slices whose fp32 partials are summed in slice order

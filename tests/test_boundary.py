@@ -6,6 +6,7 @@ import os
 import re
 import subprocess
 
+import numpy as np
 import pytest
 import torch
 
@@ -190,6 +191,36 @@ def test_key_block_plan_covers_every_key_once():
     assert sorted(blocks) == sorted([[0, 0], [1, 0], [2, 0], [2, 128], [3, 0], [3, 128], [3, 256]])
     work = [[1, 128, 129, 300][s] - k for s, k in blocks]
     assert work == sorted(work, reverse=True)  # longest work (most rows at or below the block) first
+
+
+@pytest.mark.parametrize("lens", [[2817, 301, 1, 640], [321], [448, 447], [2048] * 3 + [33]])
+def test_key_block_plan_chunks_cover_every_row_once(lens):
+    """Key blocks with more query rows than an item takes: every (key block, query row) pair is in exactly one work
+    item, no item is longer than the cap, and a split block's partial slots are its own, in row order."""
+    plan = hip_ops.KeyBlockPlan(lens, "cpu")
+    cap = plan._row_cap(lens)
+    assert cap >= hip_ops.KeyBlockPlan.MIN_ROWS and max(lens) > cap and not plan.prefixed
+    items = plan.plan.view(-1, 5).tolist()
+    assert len(items) == plan.n_blocks and [-i[3] for i in items] == sorted((-i[3] for i in items), reverse=True)
+    red = plan.reduce.tolist()
+    assert len(red) == plan.n_reduce
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    seen, slots = {}, {}
+    for seq, ks, r, nrows, slot in items:
+        assert 0 < -nrows <= cap and r >= ks and r - nrows <= lens[seq]
+        seen.setdefault((seq, ks), []).append((r, r - nrows, slot))
+    assert sorted(seen) == [(i, ks) for i, n in enumerate(lens) for ks in range(0, n, 128)]
+    for (seq, ks), parts in seen.items():
+        parts.sort()
+        assert parts[0][0] == ks and parts[-1][1] == lens[seq]
+        assert all(a[1] == b[0] for a, b in zip(parts, parts[1:]))
+        if len(parts) == 1:
+            assert parts[0][2] == -1
+        else:
+            slots[int(cu[seq]) + ks] = (min(128, lens[seq] - ks), parts[0][2], len(parts))
+            assert [p[2] for p in parts] == list(range(parts[0][2], parts[0][2] + len(parts)))
+    assert {a: (b, c, d) for a, b, c, d in red} == slots
+    assert plan.n_slots == sum(s[2] for s in slots.values())
 
 
 def _attention_plan_loops(q_lens, k_lens, causal, block=64):

@@ -65,6 +65,30 @@ def test_attention_backward(lens):
         off += n
 
 
+@pytest.mark.parametrize("lens", [[449], [1000, 65, 2817], [320, 321]])
+def test_attention_backward_split_key_blocks(lens):
+    """Key blocks whose query rows are split over several work items: the one-item-per-block gradients up to the order
+    of fp32 sums, dQ bit for bit, the same bits twice."""
+    n = sum(lens)
+    g = torch.Generator().manual_seed(n)
+    q, k, v, do = (torch.randn(n, h, 64, generator=g).to(BF).to(DEV) for h in (8, 2, 2, 8))
+    plan = TR.TrainPlan(lens, DEV)
+    assert plan.keys.n_slots > 0
+    whole = TR.TrainPlan(lens, DEV)
+    whole.keys.reduce = None
+    blocks = sorted(((m - ks, i, ks) for i, m in enumerate(lens) for ks in range(0, m, 128)), key=lambda b: -b[0])
+    whole.keys.plan = torch.tensor([x for b in blocks for x in b[1:]], dtype=torch.int32, device=DEV)
+    whole.keys.n_blocks = len(blocks)
+    lse = torch.empty(n, 8, dtype=torch.float32, device=DEV)
+    o = ops.varlen_attention(q, k, v, plan.attn, lse=lse)
+    got = ops.attention_backward(q, k, v, o, do, lse, plan.attn, plan.keys)
+    want = ops.attention_backward(q, k, v, o, do, lse, whole.attn, whole.keys)
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:], want[1:]):
+        assert float((a - b).norm() / b.norm()) < 3e-6  # sums of up to 4 n fp32 terms in another order
+    assert all(torch.equal(a, b) for a, b in zip(got, ops.attention_backward(q, k, v, o, do, lse, plan.attn, plan.keys)))
+
+
 @pytest.mark.parametrize("pre_lens,G,T", [((300, 129), 3, 100), ((64,), 2, 1), ((1000, 517), 4, 256)])
 def test_attention_backward_shared_prefix(pre_lens, G, T):
     """The shared-prefix layout (TrainPlan.shared: each group's prefix rows once, then every member's T token rows

@@ -238,7 +238,14 @@ __global__ __launch_bounds__(512) void attn_bwd_dq_kernel(
 }
 
 // ---- dK / dV: workgroup = AB_KB keys of one sequence x one KV head ----------------------------------------
-template <bool PREFIXED>
+// MODE AB_PLAIN: (sequence, first key) items; AB_PREFIXED: the items above; AB_CHUNKED: plain causal self-attention
+// whose key blocks' query rows are split into chunks, items as AB_PREFIXED's with xl < 0; slot >= 0 then names a block
+// of AB_KB partial rows of its own (part row slot * AB_KB + key - ks), summed by attn_bwd_chunk_reduce_kernel. Why
+// chunks: an item's time goes with its query rows, so the first key blocks of the longest windows set the end of a
+// launch. The whole backward (dot, dQ, dK / dV, sums): 24 windows of 301-2817 rows 512 -> 363 us, one of 2816 rows
+// 315 -> 131, four 326 -> 194, two of 900 113 -> 76; 24 of 2048 (items already even) 482 -> 477.
+enum AbMode { AB_PLAIN = 0, AB_PREFIXED = 1, AB_CHUNKED = 2 };
+template <int MODE>
 __global__ __launch_bounds__(AB_KW * 64, 2) void attn_bwd_dkdv_kernel(
     const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v,
     const bf16_t *__restrict__ dout, const float *__restrict__ lse, const float *__restrict__ dd,
@@ -251,11 +258,11 @@ __global__ __launch_bounds__(AB_KW * 64, 2) void attn_bwd_dkdv_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform for the compiler
   const int col = lane & 15, g = lane >> 4;
   const int hk = blockIdx.y;
-  constexpr int PS = PREFIXED ? 5 : 2;  // plan entry size
+  constexpr int PS = MODE != AB_PLAIN ? 5 : 2;  // plan entry size
   const int seq = plan[PS * blockIdx.x], ks = plan[PS * blockIdx.x + 1];
-  const int xl = PREFIXED ? plan[PS * blockIdx.x + 3] : -1;
-  const int64_t xr0 = PREFIXED ? plan[PS * blockIdx.x + 2] : 0;
-  const int slot = PREFIXED ? plan[PS * blockIdx.x + 4] : -1;
+  const int xl = MODE != AB_PLAIN ? plan[PS * blockIdx.x + 3] : -1;
+  const int64_t xr0 = MODE != AB_PLAIN ? plan[PS * blockIdx.x + 2] : 0;
+  const int slot = MODE != AB_PLAIN ? plan[PS * blockIdx.x + 4] : -1;
   if (seq < 0 || seq >= n_seq || ks < 0) return;
   const int64_t r0 = cu[seq];
   const int len = cu[seq + 1] - static_cast<int>(r0);
@@ -263,8 +270,8 @@ __global__ __launch_bounds__(AB_KW * 64, 2) void attn_bwd_dkdv_kernel(
   // query tiles: the sequence's own rows from the block's first key (causal), or the xl extra rows
   const bool xt = xl >= 0;  // extra rows: every row sees every key of the block
   // own rows (causal): rows r_beg .. r_lim - 1 of the sequence; extra rows: 0 .. xl - 1 from packed row xr0
-  const int r_beg = xt ? 0 : (PREFIXED ? static_cast<int>(xr0) : ks);
-  const int r_lim = xt ? xl : (PREFIXED ? min(len, r_beg - xl) : len);
+  const int r_beg = xt ? 0 : (MODE != AB_PLAIN ? static_cast<int>(xr0) : ks);
+  const int r_lim = xt ? xl : (MODE != AB_PLAIN ? min(len, r_beg - xl) : len);
   const int ntl = r_lim > r_beg ? (r_lim - r_beg + 31) / 32 : 0;
 
   // this wave's 32 keys, two blocks of 16 (lane col -> key of each), K^T / V^T fragments of the B operand
@@ -417,7 +424,9 @@ __global__ __launch_bounds__(AB_KW * 64, 2) void attn_bwd_dkdv_kernel(
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb) {
     if (keyb[kb] < len) {
-      const int64_t orow = slot < 0 ? r0 + keyb[kb] : slot * pre.n_part + r0 + keyb[kb];
+      const int64_t orow = slot < 0 ? r0 + keyb[kb]
+                                     : (MODE == AB_CHUNKED ? slot * static_cast<int64_t>(AB_KB) + keyb[kb] - ks
+                                                           : slot * pre.n_part + r0 + keyb[kb]);
       float *dkp = (slot < 0 ? dk : pre.part_k) + (orow * AB_HKV + hk) * AB_D + 4 * g;
       float *dvp = (slot < 0 ? dv : pre.part_v) + (orow * AB_HKV + hk) * AB_D + 4 * g;
 #pragma unroll
@@ -446,15 +455,46 @@ __global__ __launch_bounds__(256) void attn_bwd_part_reduce_kernel(const float *
   reinterpret_cast<f32x4 *>(dv)[i] = b;
 }
 
+// The chunked key blocks' dk / dv rows: entry (first row, keys, first slot, slots) of red sums its partial blocks in slot
+// order. blockIdx.y: a quarter of the block's 128 keys; 4 values per thread and step.
+__global__ __launch_bounds__(256) void attn_bwd_chunk_reduce_kernel(const int32_t *__restrict__ red,
+                                                                    const float *__restrict__ part_k,
+                                                                    const float *__restrict__ part_v,
+                                                                    float *__restrict__ dk, float *__restrict__ dv) {
+  constexpr int ROW4 = AB_HKV * AB_D / 4, BLK4 = AB_KB * ROW4;  // f32x4 per row / per partial block
+  const int64_t row0 = red[4 * blockIdx.x];
+  const int keys = red[4 * blockIdx.x + 1], n = red[4 * blockIdx.x + 3];
+  const int64_t slot0 = red[4 * blockIdx.x + 2];
+  const f32x4 *pk = reinterpret_cast<const f32x4 *>(part_k) + slot0 * BLK4;
+  const f32x4 *pv = reinterpret_cast<const f32x4 *>(part_v) + slot0 * BLK4;
+#pragma unroll
+  for (int it = 0; it < BLK4 / 4 / 256; ++it) {
+    const int i = blockIdx.y * (BLK4 / 4) + it * 256 + threadIdx.x;
+    if (i / ROW4 >= keys) continue;
+    f32x4 a = pk[i], b = pv[i];
+    for (int c = 1; c < n; ++c) {
+      a += pk[c * BLK4 + i];
+      b += pv[c * BLK4 + i];
+    }
+    reinterpret_cast<f32x4 *>(dk)[row0 * ROW4 + i] = a;
+    reinterpret_cast<f32x4 *>(dv)[row0 * ROW4 + i] = b;
+  }
+}
+
 }  // namespace vk
 
 using namespace vk;
 
+struct AbChunks {
+  const int32_t *red;
+  int32_t n_red;
+};
+
 static int attn_bwd_launch(const void *q, const void *k, const void *v, const void *out, const void *dout,
                            const float *lse, const int32_t *cu, int32_t n_seq, const int32_t *q_plan,
                            int32_t n_qblocks, const int32_t *k_plan, int32_t n_kblocks, int64_t n_rows,
-                           int64_t stride_tok, const AbPrefix *pre, int32_t n_slots, float *dd, float *dq,
-                           float *dk, float *dv, int32_t H, int32_t HKV, int32_t D, void *stream) {
+                           int64_t stride_tok, const AbPrefix *pre, int32_t n_slots, const AbChunks *chunks, float *dd,
+                           float *dq, float *dk, float *dv, int32_t H, int32_t HKV, int32_t D, void *stream) {
   VK_CHECK_ARG(q && k && v && out && dout && lse && cu && dd && dq && dk && dv, "attention_backward: null pointer");
   if (H != AB_H || HKV != AB_HKV || D != AB_D)
     return fail(VK_ERR_UNSUPPORTED, "attention_backward: built for H=8 HKV=2 D=64 (got %d/%d/%d)", H, HKV, D);
@@ -465,7 +505,7 @@ static int attn_bwd_launch(const void *q, const void *k, const void *v, const vo
   VK_CHECK_ARG(vk_aligned16(q) && vk_aligned16(k) && vk_aligned16(v) && vk_aligned16(out) && vk_aligned16(dout) &&
                    vk_aligned16(dq) && vk_aligned16(dk) && vk_aligned16(dv),
                "attention_backward: pointers must be 16-byte aligned");
-  VK_CHECK_ARG(pre == nullptr || (pre->p_lens && pre->p_off && pre->n_part >= 0 &&
+  VK_CHECK_ARG(pre == nullptr || chunks != nullptr || (pre->p_lens && pre->p_off && pre->n_part >= 0 &&
                                   (pre->n_part == 0 || (pre->part_k && pre->part_v && vk_aligned16(pre->part_k) &&
                                                         vk_aligned16(pre->part_v)))),
                "attention_backward_prefixed: prefix arrays or partial buffers");
@@ -485,7 +525,7 @@ static int attn_bwd_launch(const void *q, const void *k, const void *v, const vo
   if (rc != VK_OK) return rc;
   if (n_qblocks > 0) {
     const dim3 grid(static_cast<unsigned>(n_qblocks), AB_HKV);
-    if (pre != nullptr)
+    if (pre != nullptr && chunks == nullptr)
       attn_bwd_dq_kernel<true><<<grid, 512, 0, s>>>(qb, kb, vb, dob, lse, dd, cu, q_plan, n_seq, stride_tok, dq,
                                                    scale_log2, scale, *pre);
     else
@@ -496,14 +536,21 @@ static int attn_bwd_launch(const void *q, const void *k, const void *v, const vo
   }
   if (n_kblocks > 0) {
     const dim3 grid(static_cast<unsigned>(n_kblocks), AB_HKV);
-    if (pre != nullptr)
-      attn_bwd_dkdv_kernel<true><<<grid, AB_KW * 64, 0, s>>>(qb, kb, vb, dob, lse, dd, cu, k_plan, n_seq, stride_tok,
-                                                            dk, dv, scale_log2, scale, *pre);
-    else
-      attn_bwd_dkdv_kernel<false><<<grid, AB_KW * 64, 0, s>>>(qb, kb, vb, dob, lse, dd, cu, k_plan, n_seq, stride_tok,
-                                                             dk, dv, scale_log2, scale, none);
+    auto kern = chunks != nullptr ? attn_bwd_dkdv_kernel<AB_CHUNKED>
+                : pre != nullptr  ? attn_bwd_dkdv_kernel<AB_PREFIXED>
+                                  : attn_bwd_dkdv_kernel<AB_PLAIN>;
+    kern<<<grid, AB_KW * 64, 0, s>>>(qb, kb, vb, dob, lse, dd, cu, k_plan, n_seq, stride_tok, dk, dv, scale_log2, scale,
+                                     pre != nullptr ? *pre : none);
     rc = launch_status("attention_backward dkdv");
     if (rc != VK_OK) return rc;
+  }
+  if (chunks != nullptr) {
+    if (chunks->n_red > 0) {
+      attn_bwd_chunk_reduce_kernel<<<dim3(static_cast<unsigned>(chunks->n_red), 4), 256, 0, s>>>(
+          chunks->red, pre->part_k, pre->part_v, dk, dv);
+      rc = launch_status("attention_backward chunk sums");
+    }
+    return rc;
   }
   if (pre != nullptr && pre->n_part > 0 && n_slots > 0) {
     const int64_t n4 = pre->n_part * AB_HKV * AB_D / 4;
@@ -520,7 +567,7 @@ extern "C" int vk_attention_backward(const void *q, const void *k, const void *v
                                      int64_t stride_tok, float *dd, float *dq, float *dk, float *dv, int32_t H,
                                      int32_t HKV, int32_t D, void *stream) {
   return attn_bwd_launch(q, k, v, out, dout, lse, cu, n_seq, q_plan, n_qblocks, k_plan, n_kblocks, n_rows, stride_tok,
-                         nullptr, 0, dd, dq, dk, dv, H, HKV, D, stream);
+                         nullptr, 0, nullptr, dd, dq, dk, dv, H, HKV, D, stream);
 }
 
 extern "C" int vk_attention_backward_prefixed(const void *q, const void *k, const void *v, const void *out,
@@ -533,5 +580,19 @@ extern "C" int vk_attention_backward_prefixed(const void *q, const void *k, cons
   VK_CHECK_ARG(n_slots >= 0 && n_part <= n_rows, "attention_backward_prefixed: bad partial sizes");
   const AbPrefix pre{p_lens, p_off, part_k, part_v, n_part};
   return attn_bwd_launch(q, k, v, out, dout, lse, cu, n_seq, q_plan, n_qblocks, k_plan, n_kblocks, n_rows, stride_tok,
-                         &pre, n_slots, dd, dq, dk, dv, H, HKV, D, stream);
+                         &pre, n_slots, nullptr, dd, dq, dk, dv, H, HKV, D, stream);
+}
+
+extern "C" int vk_attention_backward_chunked(const void *q, const void *k, const void *v, const void *out,
+                                             const void *dout, const float *lse, const int32_t *cu, int32_t n_seq,
+                                             const int32_t *q_plan, int32_t n_qblocks, const int32_t *k_plan,
+                                             int32_t n_kblocks, int64_t n_rows, int64_t stride_tok, const int32_t *red,
+                                             int32_t n_red, float *part_k, float *part_v, float *dd, float *dq,
+                                             float *dk, float *dv, int32_t H, int32_t HKV, int32_t D, void *stream) {
+  VK_CHECK_ARG(n_red >= 0 && (n_red == 0 || (red && part_k && part_v && vk_aligned16(part_k) && vk_aligned16(part_v))),
+               "attention_backward_chunked: partial buffers");
+  const AbPrefix pre{nullptr, nullptr, part_k, part_v, 0};
+  const AbChunks chunks{red, n_red};
+  return attn_bwd_launch(q, k, v, out, dout, lse, cu, n_seq, q_plan, n_qblocks, k_plan, n_kblocks, n_rows, stride_tok,
+                         &pre, 0, &chunks, dd, dq, dk, dv, H, HKV, D, stream);
 }

@@ -605,6 +605,8 @@ class KeyBlockPlan:
     (most query rows at or below the block) first: the dK / dV work list of attention_backward."""
 
     BLOCK = 128
+    MIN_ROWS = 320   # of a work item whose key block is split
+    RESIDENT = 512   # workgroups of the dK / dV kernel on the chip: two per CU
 
     def __init__(self, seq_lens, device, extra=None, chunk=None):
         """extra (the shared-prefix layout of vk_attention_backward_prefixed): per sequence, a list of (first
@@ -615,7 +617,12 @@ class KeyBlockPlan:
         packing and carry the same number of segments."""
         lens = [int(n) for n in seq_lens]
         self.n_slots, self.n_part = 0, 0
-        self.part = None
+        self.part = self.reduce = None
+        cap = self._row_cap(lens) if extra is None else 0
+        self.prefixed = extra is not None
+        if extra is None and max(lens, default=0) > cap:
+            self._chunked(lens, cap, device)
+            return
         if extra is None:
             blocks = sorted(((n - ks, i, ks) for i, n in enumerate(lens) for ks in range(0, n, self.BLOCK)),
                             key=lambda b: -b[0])
@@ -647,8 +654,38 @@ class KeyBlockPlan:
             flat = [v for it in items for v in it[1:]] or [0, 0, 0, -1, -1]
             blocks = items
         self.n_blocks = len(blocks)
-        self.prefixed = extra is not None
         self.plan = torch.tensor(flat, dtype=torch.int32).to(device)
+
+    def _row_cap(self, lens):
+        """The most query rows of one work item: the share of a resident workgroup (two per CU, one per KV head of an
+        item), so no item outlasts the launch's mean; at least MIN_ROWS, below which the partial sums cost more."""
+        rows = sum(nb * n - self.BLOCK * (nb * (nb - 1) // 2) for n in lens for nb in [-(-n // self.BLOCK)])
+        return max(self.MIN_ROWS, -(-2 * rows // (self.RESIDENT * 32)) * 32)
+
+    def _chunked(self, lens, cap, device):
+        """The plan of work items (sequence, first key, first row, -rows, slot), longest first: blocks with more than cap
+        query rows in even chunks with a partial slot each, and the list of those blocks (vk_attention_backward_chunked)."""
+        n = np.asarray(lens, dtype=np.int64)
+        cu = np.cumsum(n) - n
+        nb = -(-n // self.BLOCK)
+        seq = np.repeat(np.arange(len(n)), nb)
+        ks = (np.arange(len(seq)) - np.repeat(np.cumsum(nb) - nb, nb)) * self.BLOCK
+        rows = n[seq] - ks
+        size = -(-rows // (32 * -(-rows // cap))) * 32
+        parts = -(-rows // size)
+        split = parts > 1
+        slots = np.where(split, parts, 0)
+        slot0 = np.cumsum(slots) - slots
+        at = np.repeat(np.arange(len(seq)), parts)
+        j = np.arange(len(at)) - np.repeat(np.cumsum(parts) - parts, parts)
+        r = ks[at] + j * size[at]
+        count = np.minimum(size[at], n[seq[at]] - r)
+        items = np.stack([seq[at], ks[at], r, -count, np.where(split[at], slot0[at] + j, -1)], 1)
+        items = items[np.argsort(-count, kind="stable")]
+        red = np.stack([cu[seq] + ks, np.minimum(self.BLOCK, rows), slot0, parts], 1)[split]
+        self.n_slots, self.n_reduce, self.n_blocks = int(slots.sum()), len(red), len(items)
+        both = torch.from_numpy(np.concatenate([items.reshape(-1), red.reshape(-1)]).astype(np.int32)).to(device)
+        self.plan, self.reduce = both[:items.size], both[items.size:].view(-1, 4)
 
     def partials(self, hkv, d, device):
         """The plan's partial-slot workspace (k, v) [n_slots, n_part, hkv, d] fp32, zeroed once: every call with
@@ -682,6 +719,13 @@ def attention_backward(q, k, v, out, dout, lse, q_plan: AttentionPlan, k_plan: K
     dk = torch.empty(n, HK, D, dtype=torch.float32, device=q.device)
     dv = torch.empty_like(dk)
     prefixed = q_plan.p_lens is not None or k_plan.prefixed
+    if not prefixed and k_plan.reduce is not None:
+        part = torch.empty(2, k_plan.n_slots, k_plan.BLOCK, HK, D, dtype=torch.float32, device=q.device)
+        call("vk_attention_backward_chunked", ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), ptr(lse), ptr(q_plan.cu_q),
+             q_plan.n_seq, ptr(q_plan.plan), q_plan.n_blocks, ptr(k_plan.plan), k_plan.n_blocks, n, stride_tok,
+             ptr(k_plan.reduce), k_plan.n_reduce, ptr(part[0]), ptr(part[1]), ptr(dd), ptr(dq), ptr(dk), ptr(dv), H, HK, D,
+             stream_handle())
+        return dq, dk, dv
     if not prefixed:
         call("vk_attention_backward", ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), ptr(lse), ptr(q_plan.cu_q),
              q_plan.n_seq, ptr(q_plan.plan), q_plan.n_blocks, ptr(k_plan.plan), k_plan.n_blocks, n, stride_tok,
