@@ -674,6 +674,32 @@ def test_greedy_update_reference_signature():
             assert int(oc[b, c]) == int(want_tok[b])
 
 
+@pytest.mark.parametrize("T", [1, 255, 256, 257, 1024, 1025])
+@pytest.mark.parametrize("V,dtype", [(1, torch.float32), (7, BF), (8, torch.float32), (9, BF)])
+def test_gspo_score_few_logits(V, T, dtype):
+    """The kernel that keeps a row's logits in registers, at the edges of its rounds and of its range (T = 1025 and V = 9
+    run the one that reads them twice), against fp64: 1e-5 for fp32 exponentials and sums of T terms."""
+    g = gen(T + V)
+    B = 3
+    z = to_dev(torch.randn(B, T, V, generator=g), dtype)
+    y = torch.randint(-1, V, (B, T), generator=g).to(DEV)
+    mask = (torch.rand(B, T, generator=g) > 0.3).to(DEV)
+    mask[:, 0] = True
+    z64 = z.double().requires_grad_()
+    lp64 = torch.log_softmax(z64, -1).gather(-1, y.clamp(min=0)[..., None])[..., 0]
+    old = (lp64.detach() + 1e-3 * to_dev(torch.randn(B, T, generator=g)).double()).float()
+    nb = torch.full((B,), float(T), device=DEV)
+    adv = torch.tensor([1.0, -0.5, 0.25], device=DEV)
+    s64 = torch.exp(((lp64 - old.double()) * mask).sum(-1) / T)
+    pg64 = -torch.minimum(s64 * adv, s64.clamp(1 - 0.2, 1 + 0.2) * adv)
+    pg64.mean().backward()
+    res = ops.gspo_score(z, y, mask, old, nb, adv, 0.2, 0.2)
+    assert torch.allclose(res["lp"].double(), lp64, rtol=1e-5, atol=1e-5)
+    assert torch.allclose(res["s"].double(), s64, rtol=1e-5) and torch.allclose(res["pg"].double(), pg64, rtol=1e-5)
+    assert torch.allclose(res["dlogits"].double(), z64.grad, rtol=1e-4, atol=1e-5 / T)
+    assert torch.equal(ops.gspo_score(z, y)["lp"], res["lp"])
+
+
 @pytest.mark.parametrize("V,dtype", [(7, torch.float32), (7, BF), (343, BF)])
 def test_gspo_score(V, dtype):
     g = gen(V)

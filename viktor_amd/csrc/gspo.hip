@@ -57,6 +57,105 @@ __device__ __forceinline__ float block_sum(float v, float *scratch) {
   return t;
 }
 
+// From the masked sum of a sequence: its ratio and objective, and (returned) the factor of its logits' gradient.
+__device__ __forceinline__ float ratio_terms(float tot, float nb, float A, float eps_lo, float eps_hi, float inv_n,
+                                             float *s_out, float *pg_out) {
+  const float s = expf(tot / nb);
+  const float lo = 1.0f - eps_lo, hi = 1.0f + eps_hi;
+  const float sc = fminf(fmaxf(s, lo), hi);
+  const float a1 = s * A, a2 = sc * A;
+  *s_out = s;
+  *pg_out = -fminf(a1, a2);
+  // d min(a1, a2) / ds: a1 branch slope A, a2 branch slope A * [lo <= s <= hi]; ties split evenly
+  const float d2 = (s >= lo && s <= hi) ? A : 0.f;
+  float dmin;
+  if (a1 < a2)
+    dmin = A;
+  else if (a2 < a1)
+    dmin = d2;
+  else
+    dmin = 0.5f * (A + d2);
+  const float g = -dmin;
+  return inv_n * g * s / nb;
+}
+
+// Vocabularies of at most GS_V logits and T <= GS_THREADS * GS_TPT: a token per thread and round, its logits in
+// registers from the log-probs to the gradient. Bound by memory: rows of V elements are no vectors (V = 7), so a
+// round's logits and gradients go through LDS and its global accesses are consecutive over the lanes. 512 x 1024
+// tokens of 7 bf16 logits with the gradient: 31 us (every token's logits read and exponentiated twice by strided
+// 2-byte loads) -> 24 us.
+constexpr int GS_V = 8, GS_TPT = 4;
+template <bool BF16>
+__global__ __launch_bounds__(GS_THREADS) void gspo_score_few_kernel(
+    const void *__restrict__ logits, const int64_t *__restrict__ targets, const uint8_t *__restrict__ mask,
+    const float *__restrict__ old_lp, const float *__restrict__ n_bases, const float *__restrict__ adv, float eps_lo,
+    float eps_hi, float inv_n, float *__restrict__ lp_out, float *__restrict__ s_out, float *__restrict__ pg_out,
+    float *__restrict__ dlogits, int T, int V) {
+  __shared__ float scratch[GS_THREADS / 64];
+  __shared__ float coef_sh;
+  __shared__ float stage[GS_THREADS * GS_V];
+  const int64_t b = blockIdx.x;
+  const int tid = threadIdx.x;
+  const bool ratio = old_lp != nullptr && adv != nullptr && n_bases != nullptr;
+  float z[GS_TPT][GS_V], lse[GS_TPT];
+  int yv[GS_TPT];
+  bool on[GS_TPT];
+  float part = 0.f;
+#pragma unroll
+  for (int c = 0; c < GS_TPT; ++c) {
+    const int t0 = c * GS_THREADS, t = t0 + tid;
+    if (t0 >= T) break;  // uniform
+    const int n = min(GS_THREADS, T - t0) * V;
+    __syncthreads();  // the previous round's readers are done
+    for (int i = tid; i < n; i += GS_THREADS) stage[i] = logit_at<BF16>(logits, (b * T + t0) * V + i);
+    __syncthreads();
+    on[c] = false;
+    if (t >= T) continue;
+    const int64_t row = b * T + t;
+    int64_t y = targets[row];
+    y = (y < 0 || y >= V) ? 0 : y;
+    yv[c] = static_cast<int>(y);
+    float mx = -INFINITY, s = 0.f;
+#pragma unroll
+    for (int v = 0; v < GS_V; ++v) {
+      z[c][v] = v < V ? stage[tid * V + v] : -INFINITY;
+      if (v < V) mx = fmaxf(mx, z[c][v]);
+    }
+#pragma unroll
+    for (int v = 0; v < GS_V; ++v)
+      if (v < V) s += expf(z[c][v] - mx);
+    lse[c] = mx + logf(s);
+    const float lp = stage[tid * V + yv[c]] - lse[c];
+    lp_out[row] = lp;
+    if (ratio) {
+      on[c] = mask[row] != 0;
+      if (on[c]) part += lp - old_lp[row];
+    }
+  }
+  if (!ratio) return;
+  const float tot = block_sum(part, scratch);
+  if (tid == 0) coef_sh = ratio_terms(tot, n_bases[b], adv[b], eps_lo, eps_hi, inv_n, s_out + b, pg_out + b);
+  if (dlogits == nullptr) return;
+  __syncthreads();
+  const float coef = coef_sh;
+  // dL/dz = coef * mask * (onehot - softmax)
+#pragma unroll
+  for (int c = 0; c < GS_TPT; ++c) {
+    const int t0 = c * GS_THREADS;
+    if (t0 >= T) break;
+    const int n = min(GS_THREADS, T - t0) * V;
+    const float k = on[c] ? coef : 0.f;
+    if (t0 + tid < T) {
+#pragma unroll
+      for (int v = 0; v < GS_V; ++v)
+        if (v < V) stage[tid * V + v] = k * ((v == yv[c] ? 1.f : 0.f) - expf(z[c][v] - lse[c]));
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += GS_THREADS) dlogits[(b * T + t0) * V + i] = stage[i];
+    __syncthreads();
+  }
+}
+
 template <bool BF16, bool WAVE_PER_TOKEN>
 __global__ __launch_bounds__(GS_THREADS) void gspo_score_kernel(
     const void *__restrict__ logits, const int64_t *__restrict__ targets, const uint8_t *__restrict__ mask,
@@ -90,27 +189,7 @@ __global__ __launch_bounds__(GS_THREADS) void gspo_score_kernel(
   }
   if (!ratio) return;
   const float tot = block_sum(part, scratch);
-  if (tid == 0) {
-    const float nb = n_bases[b];
-    const float A = adv[b];
-    const float s = expf(tot / nb);
-    const float lo = 1.0f - eps_lo, hi = 1.0f + eps_hi;
-    const float sc = fminf(fmaxf(s, lo), hi);
-    const float a1 = s * A, a2 = sc * A;
-    s_out[b] = s;
-    pg_out[b] = -fminf(a1, a2);
-    // d min(a1, a2) / ds: a1 branch slope A, a2 branch slope A * [lo <= s <= hi]; ties split evenly
-    const float d2 = (s >= lo && s <= hi) ? A : 0.f;
-    float dmin;
-    if (a1 < a2)
-      dmin = A;
-    else if (a2 < a1)
-      dmin = d2;
-    else
-      dmin = 0.5f * (A + d2);
-    const float g = -dmin;
-    coef_sh = inv_n * g * s / nb;
-  }
+  if (tid == 0) coef_sh = ratio_terms(tot, n_bases[b], adv[b], eps_lo, eps_hi, inv_n, s_out + b, pg_out + b);
   if (dlogits == nullptr) return;
   __syncthreads();
   const float coef = coef_sh;
@@ -187,7 +266,12 @@ extern "C" int vk_gspo_score(const void *logits, int32_t logits_dtype, const int
   gspo_score_kernel<BF, WV><<<grid, GS_THREADS, 0, st>>>(logits, targets, mask, ratio ? old_lp : nullptr, n_bases, \
                                                          ratio ? adv : nullptr, eps_lo, eps_hi, inv_n, lp, s, pg,   \
                                                          dlogits, T, V)
-  if (logits_dtype == VK_DTYPE_BF16) {
+  // few logits per token and rows short enough to stay in registers; longer rows read their logits twice
+  if (V <= GS_V && T <= GS_THREADS * GS_TPT) {
+    auto kern = logits_dtype == VK_DTYPE_BF16 ? gspo_score_few_kernel<true> : gspo_score_few_kernel<false>;
+    kern<<<grid, GS_THREADS, 0, st>>>(logits, targets, mask, ratio ? old_lp : nullptr, n_bases, ratio ? adv : nullptr,
+                                      eps_lo, eps_hi, inv_n, lp, s, pg, dlogits, static_cast<int>(T), V);
+  } else if (logits_dtype == VK_DTYPE_BF16) {
     if (wave)
       VK_GSPO_LAUNCH(true, true);
     else

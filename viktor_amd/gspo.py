@@ -109,12 +109,14 @@ class _GspoLoss(torch.autograd.Function):
         # the kernel's gradient is that of the loss only: s, pg and lp are outputs to read, not to backpropagate
         # through (a backward from them raises instead of returning zeros)
         ctx.mark_non_differentiable(res["s"], res["pg"], res["lp"])
+        ctx.set_materialize_grads(False)  # (three zero-filled tensors per backward otherwise)
         return res["loss"], res["s"], res["pg"], res["lp"]
 
     @staticmethod
     def backward(ctx, g_loss, g_s, g_pg, g_lp):
         (dl,) = ctx.saved_tensors
-        return (dl * g_loss).to(ctx.logits_dtype), None, None, None, None, None, None, None, None
+        dz = None if g_loss is None else (dl * g_loss).to(ctx.logits_dtype)
+        return dz, None, None, None, None, None, None, None, None
 
 
 def sequence_ratio_loss(logits, targets, mask, old_lp, n_bases, adv, eps_lo=4e-4, eps_hi=4e-4, inv_n=None):
@@ -124,5 +126,6 @@ def sequence_ratio_loss(logits, targets, mask, old_lp, n_bases, adv, eps_lo=4e-4
     Reference: scripts/gspo.py:474-477."""
     B = logits.shape[0]
     inv = 1.0 / B if inv_n is None else inv_n
-    return _GspoLoss.apply(logits, targets.clamp(min=0).contiguous(), mask, old_lp.contiguous(), n_bases, adv,
+    # (the kernel reads a negative target as 0, so PAD targets need no clamp of their own)
+    return _GspoLoss.apply(logits, targets.contiguous(), mask, old_lp.contiguous(), n_bases, adv,
                            eps_lo, eps_hi, inv)

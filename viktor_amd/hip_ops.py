@@ -567,7 +567,7 @@ def gspo_score(logits, targets, mask=None, old_lp=None, n_bases=None, adv=None, 
         _require(old_lp.shape == (B, T) and old_lp.dtype == torch.float32 and old_lp.is_contiguous(), "gspo_score: old_lp")
         _require(mask.shape == (B, T), "gspo_score: mask")
         _require(n_bases.shape == (B,) and adv.shape == (B,), "gspo_score: n_bases / adv")
-        m8 = mask.to(torch.uint8).contiguous()
+        m8 = mask.contiguous().view(torch.uint8) if mask.dtype == torch.bool else mask.to(torch.uint8).contiguous()
         n_bases = n_bases.to(torch.float32).contiguous()
         adv = adv.to(torch.float32).contiguous()
         s = torch.empty(B, dtype=torch.float32, device=dev)
