@@ -1071,6 +1071,45 @@ def test_norm_linear(M, mode):
     assert ok, err
 
 
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 31, 32, 33])
+def test_few_row_products(M):
+    """The products of at most 16 (o + residual) / 32 (gate_up + SwiGLU) rows at the edges of their row blocks, with a
+    ragged count of column blocks: the oracle's rounding points, rows past M untouched, the same bits for a row of a
+    larger call that runs the same kernel."""
+    g = gen(M + 5)
+    K = 512
+    a = R.bf(torch.randn(M, K, generator=g))
+    w = R.bf(torch.randn(96, K, generator=g) / math.sqrt(K))
+    x = R.bf(torch.randn(M + 1, 96, generator=g) * 2)
+    xd = to_dev(x, BF)
+    ops.linear_residual(to_dev(a, BF), to_dev(w, BF), xd[:M])
+    want = R.bf(x[:M] + R.bf((a.double() @ w.double().t()).float()))
+    ok, err = bf_close(xd[:M], want, ulps=1, atol=2e-2)  # (atol: as test_linear_residual)
+    assert ok, err
+    assert torch.equal(xd[M].float().cpu(), x[M])
+    nw = R.bf(torch.rand(K, generator=g) + 0.5)
+    wg = R.bf(torch.randn(2 * 48, K, generator=g) / math.sqrt(K))
+    r = R.bf(torch.randn(M, K, generator=g) * 3)
+    out = ops.norm_linear(to_dev(r, BF), to_dev(nw, BF), 1e-6, to_dev(wg, BF), swiglu=True, ss=to_dev(_row_ss(r)))
+    y = (R.rmsnorm_fused(r, nw, 1e-6).double() @ wg.double().t()).float()
+    ok, err = bf_close(out, R.swiglu_fused(R.bf(y[:, :48]), R.bf(y[:, 48:])), ulps=4, atol=3e-3)  # as test_norm_linear
+    assert ok, err
+    one = ops.norm_linear(to_dev(r[:1].contiguous(), BF), to_dev(nw, BF), 1e-6, to_dev(wg, BF), swiglu=True,
+                          ss=to_dev(_row_ss(r[:1])))
+    assert M > 32 or torch.equal(one[0], out[0])
+
+
+@pytest.mark.parametrize("B,S", [(1, 33), (1, 17 * 256 + 5), (2, 70 * 256 + 31), (3, 512)])
+def test_decode_attention_split_merge(B, S):
+    """The merge of 1 to more than 64 key splits, with sequences that reach only some of them."""
+    torch.manual_seed(S)
+    lens = torch.tensor([S, 1, 257])[:B].int()
+    q = torch.randn(B, 8, 64).to(BF)
+    k, v = torch.randn(B, S, 2, 64).to(BF), torch.randn(B, S, 2, 64).to(BF)
+    out = ops.decode_attention(q.to(DEV), k.to(DEV), v.to(DEV), lens.to(DEV))
+    assert (out.float().cpu() - _sdpa_ref(q, k, v, lens)).abs().max() < 1e-2
+
+
 def test_select_update_with_final_norm():
     g = gen(99)
     B, d, V = 64, 512, 7

@@ -73,12 +73,14 @@ __global__ __launch_bounds__(DA_WAVES * 64) void decode_attn_kernel(
   // cache row of sequence b (rows == NULL: row b); a row outside the cache gives a zero output (the
   // combine kernel writes it when the key range is split)
   const int64_t crow = rows ? static_cast<int64_t>(rows[b]) : b;
+  int64_t len = lengths[b];
+  // (both loads go out ahead of the checks: the compiler would sink the second behind the first's round trip)
+  asm volatile("" ::"s"(crow), "s"(len));
   if (crow < 0 || crow >= cache_rows) {
     if (!SPLIT && split == 0)
       for (int o = threadIdx.x; o < DA_H * DA_D; o += DA_WAVES * 64) out[b * DA_H * DA_D + o] = 0;
     return;  // uniform over the workgroup
   }
-  int64_t len = lengths[b];
   len = len < 1 ? 1 : (len > max_len ? max_len : len);
   const int ntiles = static_cast<int>((len + DA_TILE - 1) / DA_TILE);
   const int t_begin = split * tps;
@@ -260,14 +262,34 @@ __global__ __launch_bounds__(DA_H * DA_D) void decode_attn_combine(const float *
   len = len < 1 ? 1 : (len > max_len ? max_len : len);
   const int ntiles = static_cast<int>((len + DA_TILE - 1) / DA_TILE);
   const int nvalid = min(nsplit, (ntiles + tps - 1) / tps);
-  float M = -INFINITY;
-  for (int s = 0; s < nvalid; ++s) M = fmaxf(M, ws_ml[((b * nsplit + s) * DA_H + h) * 2]);
-  float L = 0.f, N = 0.f;
-  for (int s = 0; s < nvalid; ++s) {
-    const int64_t base = (b * nsplit + s) * DA_H + h;
-    const float e = exp2f(ws_ml[base * 2] - M);
-    L += e * ws_ml[base * 2 + 1];
-    N += e * ws_o[base * DA_D + d];
+  // a wavefront per head: lane s holds split s's (max, sum), 64 splits at a time, and eight splits' outputs are in
+  // flight at once (one split after another, each behind two round trips: 5.5 -> 4.6 us for 9 splits)
+  const int lane = threadIdx.x & 63;
+  float M = -INFINITY, L = 0.f, N = 0.f;
+  for (int s0 = 0; s0 < nvalid; s0 += 64) {
+    const int n = min(64, nvalid - s0);
+    const int64_t base = (b * nsplit + s0) * DA_H + h;
+    const int64_t mine = base + static_cast<int64_t>(min(lane, n - 1)) * DA_H;
+    const float m_l = ws_ml[mine * 2], l_l = ws_ml[mine * 2 + 1];
+    constexpr int U = 8;
+    float o[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) o[u] = ws_o[(base + static_cast<int64_t>(min(u, n - 1)) * DA_H) * DA_D + d];
+    const float m_new = fmaxf(M, wave_max(m_l));
+    const float keep = exp2f(M - m_new);
+    const float e_l = lane < n ? exp2f(m_l - m_new) : 0.f;
+    L = L * keep + wave_sum(e_l * l_l);
+    N *= keep;
+    M = m_new;
+    for (int s = 0; s < n; s += U) {
+      float nx[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) nx[u] = ws_o[(base + static_cast<int64_t>(min(s + U + u, n - 1)) * DA_H) * DA_D + d];
+#pragma unroll
+      for (int u = 0; u < U; ++u) N += __shfl(e_l, min(s + u, 63), 64) * (s + u < n ? o[u] : 0.f);
+#pragma unroll
+      for (int u = 0; u < U; ++u) o[u] = nx[u];
+    }
   }
   out[(b * DA_H + h) * DA_D + d] = f2bf(N / L);
 }
