@@ -33,6 +33,7 @@ extern "C" {
 
 #define VK_DTYPE_BF16 0
 #define VK_DTYPE_F32 1
+#define VK_DTYPE_F32_BF16 2 /* fp32 storage of values rounded to bf16 (vk_wgrad) */
 
 /* Library version (major * 10000 + minor * 100 + patch). */
 int vk_version(void);
@@ -398,7 +399,8 @@ int vk_attention_backward_chunked(const void *q, const void *k, const void *v, c
  * Weight gradient of a linear layer over packed rows: out[Ka, Kb] = a^T b = sum_r a[r, ka] b[r, kb] for a [N, Ka]
  * (the layer's output gradient) and b [N, Kb] (its input), bf16 row-major with row strides lda / ldb (elements,
  * multiples of 8); fp32 accumulation, the N rows split into slices whose fp32 partials are summed in slice order
- * (deterministic), then rounded to bf16 (out_dtype VK_DTYPE_BF16, the autocast matmul output) or kept fp32.
+ * (deterministic), then rounded to bf16 (out_dtype VK_DTYPE_BF16, the autocast matmul output), kept fp32, or
+ * (VK_DTYPE_F32_BF16) rounded to bf16 and stored as fp32 (that output added to an fp32 master gradient).
  * Ka % 256 == 0, Kb % 128 == 0; workspace: vk_wgrad_workspace() bytes.
  * Replaces the weight-gradient products of nn.Linear under autocast in the update's backward
  * (viktor/decoder.py:58-59, 114-115, viktor/model.py:35 differentiated by loss.backward(), scripts/gspo.py:477).
@@ -455,6 +457,15 @@ int vk_rmsnorm_backward_blocks(int64_t n, int32_t *blocks);
 int vk_rmsnorm_backward(const void *x, int32_t x_dtype, const void *w, int32_t w_dtype, const void *dy,
                         int32_t dy_dtype, const float *dres, float *dx, void *dx_bf16, float *dw_part, int64_t n,
                         int32_t d, float eps, void *stream);
+
+/*
+ * n matrices [rows[i], cols[i]] (contiguous, 16-byte aligned, rows and columns multiples of 8; the pointer and size
+ * arrays are read on the host): transpose == 0: dst[i] = bf16(src[i]) of fp32 src[i]; else dst[i] [cols, rows] = the
+ * transpose of bf16 src[i]. The casts of the fp32 master weights under torch.autocast bf16 and the transposes the
+ * update's backward products take (viktor/decoder.py:58-59, 114-115), all in one launch per 64 matrices.
+ */
+int vk_weights_bf16(const void *const *src, void *const *dst, const int32_t *rows, const int32_t *cols, int32_t n,
+                    int32_t transpose, void *stream);
 
 /* out[c] = sum_r part[r, c] (+ out[c] when accumulate), fixed order. */
 int vk_colsum(const float *part, float *out, int32_t rows, int32_t cols, int32_t accumulate, void *stream);

@@ -441,6 +441,38 @@ def test_gspo_update_steps_move_weights():
     #                                     does nothing only at step 1, so allow one untouched tensor)
 
 
+@pytest.mark.parametrize("shapes", [[(8, 8)], [(64, 64), (72, 200), (3072, 512), (512, 1536)], [(16, 72)] * 70])
+def test_weights_cast_and_transpose(shapes):
+    """All matrices in one launch (70: two), sizes that are no multiples of the 64 x 64 tile: the bits of the tensor
+    casts and transposes; a matrix the kernel does not take (7 rows, a strided view) goes the tensor way."""
+    g = gen(len(shapes))
+    ws = [torch.randn(r, c, generator=g).to(DEV) for r, c in shapes]
+    wb = ops.weights_bf16(ws)
+    assert all(torch.equal(b, w.to(BF)) for b, w in zip(wb, ws))
+    assert all(torch.equal(t, b.t()) and t.is_contiguous() for t, b in zip(ops.weights_t(wb), wb))
+    for odd in (torch.randn(7, 64, generator=g).to(DEV), torch.randn(64, 64, generator=g).to(DEV).t()):
+        b = ops.weights_bf16([ws[0], odd])
+        assert torch.equal(b[1], odd.to(BF)) and torch.equal(ops.weights_t([b[0], odd.to(BF)])[1], odd.to(BF).t())
+    assert ops.weights_bf16([]) == [] and ops.weights_t([]) == []
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 16), (63, 512), (64, 7), (513, 128), (1024, 512), (1037, 33)])
+def test_colsum(rows, cols):
+    x = torch.randn(rows, cols, generator=gen(rows)).to(DEV)
+    out = ops.colsum(x)
+    # fp32 sums of `rows` N(0, 1) terms
+    assert bool(((out.double() - x.double().sum(0)).abs() <= 2.0 ** -20 * x.double().abs().sum(0)).all())
+    assert torch.equal(ops.colsum(x, out=out.clone(), accumulate=True), out + out)
+
+
+@pytest.mark.parametrize("n", [33, 4096])
+def test_wgrad_widened(n):
+    g = gen(n)
+    a, b = (torch.randn(n, k, generator=g).to(BF).to(DEV) for k in (256, 128))
+    w = ops.wgrad(a, b, widen=True)
+    assert w.dtype == torch.float32 and torch.equal(w, ops.wgrad(a, b).float())
+
+
 @pytest.mark.parametrize("n,ka,kb", [(90112, 3072, 512), (90112, 512, 1536), (4099, 512, 512), (33, 768, 512),
                                      (1000, 256, 128), (64 * 1024 + 17, 768, 512)])
 def test_wgrad_kernel_against_fp64(n, ka, kb):

@@ -17,6 +17,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libviktor_h
 VK_OK = 0
 VK_DTYPE_BF16 = 0
 VK_DTYPE_F32 = 1
+VK_DTYPE_F32_BF16 = 2
 
 _P = ctypes.c_void_p
 _I32 = ctypes.c_int32
@@ -58,6 +59,7 @@ SIGNATURES = {
                                       _P, _P, _P, _P, _I32, _I32, _I32, _P],
     "vk_attention_backward_prefixed": [_P, _P, _P, _P, _P, _P, _P, _I32, _P, _I32, _P, _I32, _I64, _I64, _P, _P, _P,
                                        _P, _I64, _I32, _P, _P, _P, _P, _I32, _I32, _I32, _P],
+    "vk_weights_bf16": [_P, _P, _P, _P, _I32, _I32, _P],
     "vk_wgrad": [_P, _I64, _P, _I64, _I64, _I32, _I32, _P, _I32, _P, _I64, _P],
     "vk_wgrad_workspace": [_I64, _I32, _I32, ctypes.POINTER(_I64)],
     "vk_bias_act": [_P, _P, _P, _P, _I64, _I32, _I32, _P],

@@ -188,14 +188,19 @@ __global__ __launch_bounds__((WG_CONS + WG_PROD) * 64, 1) void wgrad_kernel(
   }
 }
 
-// out[c] = sum over slices s (in order) of ws[s, c], rounded to bf16 (out_bf16) or kept fp32; 4 columns a thread.
+// out[c] = sum over slices s (in order) of ws[s, c], rounded to bf16 (VK_DTYPE_BF16), kept fp32, or
+// (VK_DTYPE_F32_BF16) rounded to bf16 and stored as fp32; 4 columns a thread.
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restrict__ ws, int slices, int64_t n,
-                                                           void *__restrict__ out, int out_bf16) {
+                                                           void *__restrict__ out, int out_dtype) {
   const int64_t c = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (c >= n) return;
   f32x4 acc = *reinterpret_cast<const f32x4 *>(ws + c);
   for (int s = 1; s < slices; ++s) acc += *reinterpret_cast<const f32x4 *>(ws + static_cast<int64_t>(s) * n + c);
-  if (out_bf16)
+  if (out_dtype == VK_DTYPE_F32_BF16) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = round_bf(acc[e]);
+  }
+  if (out_dtype == VK_DTYPE_BF16)
     *reinterpret_cast<u32x2 *>(static_cast<bf16_t *>(out) + c) = u32x2{pack_bf(acc[0], acc[1]), pack_bf(acc[2], acc[3])};
   else
     *reinterpret_cast<f32x4 *>(static_cast<float *>(out) + c) = acc;
@@ -232,7 +237,8 @@ extern "C" int vk_wgrad(const void *a, int64_t lda, const void *b, int64_t ldb, 
   VK_CHECK_ARG(lda >= Ka && ldb >= Kb && lda % 8 == 0 && ldb % 8 == 0, "wgrad: row strides (multiples of 8, >= width)");
   VK_CHECK_ARG(vk_aligned16(a) && vk_aligned16(b) && vk_aligned16(out) && vk_aligned16(workspace),
                "wgrad: 16-byte aligned operands");
-  VK_CHECK_ARG(out_dtype == VK_DTYPE_BF16 || out_dtype == VK_DTYPE_F32, "wgrad: bad out dtype");
+  VK_CHECK_ARG(out_dtype == VK_DTYPE_BF16 || out_dtype == VK_DTYPE_F32 || out_dtype == VK_DTYPE_F32_BF16,
+               "wgrad: bad out dtype");
   const int tiles_kb = Kb / WG_BI, tiles = (Ka / WG_BJ) * tiles_kb;
   const int slices = wgrad_slices(N, tiles, device_cus_cached());
   const int64_t need = static_cast<int64_t>(slices) * Ka * Kb * static_cast<int64_t>(sizeof(float));
@@ -248,6 +254,6 @@ extern "C" int vk_wgrad(const void *a, int64_t lda, const void *b, int64_t ldb, 
   if (rc != VK_OK) return rc;
   const int64_t n = static_cast<int64_t>(Ka) * Kb;
   wgrad_reduce_kernel<<<static_cast<unsigned>((n / 4 + 255) / 256), 256, 0, s>>>(
-      static_cast<const float *>(workspace), slices, n, out, out_dtype == VK_DTYPE_BF16);
+      static_cast<const float *>(workspace), slices, n, out, out_dtype);
   return launch_status("wgrad reduce");
 }

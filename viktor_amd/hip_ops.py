@@ -21,7 +21,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import VK_DTYPE_BF16, VK_DTYPE_F32, call, ptr, require_device, stream_handle
+from ._lib import VK_DTYPE_BF16, VK_DTYPE_F32, VK_DTYPE_F32_BF16, call, ptr, require_device, stream_handle
 
 BF16 = torch.bfloat16
 
@@ -746,10 +746,10 @@ def attention_backward(q, k, v, out, dout, lse, q_plan: AttentionPlan, k_plan: K
 _wgrad_ws = {}
 
 
-def wgrad(a, b, out_dtype=BF16):
+def wgrad(a, b, out_dtype=BF16, widen=False):
     """Weight gradient a^T b [Ka, Kb] over the rows of a [N, Ka] and b [N, Kb] (bf16, unit column stride):
-    fp32 accumulation in row slices summed in a fixed order, rounded to bf16 once (or fp32). Ka % 256 == 0,
-    Kb % 128 == 0. The workspace is cached per (N, Ka, Kb, device)."""
+    fp32 accumulation in row slices summed in a fixed order, rounded to bf16 once (or fp32). widen: the bf16 result
+    in an fp32 tensor, as .float() of it. Ka % 256 == 0, Kb % 128 == 0. The workspace is cached per (N, Ka, Kb, device)."""
     require_device(a, "wgrad")
     _require(a.dim() == 2 and b.dim() == 2 and a.shape[0] == b.shape[0] and a.dtype == b.dtype == BF16,
              "wgrad: a [N, Ka], b [N, Kb] bf16")
@@ -765,10 +765,44 @@ def wgrad(a, b, out_dtype=BF16):
         if len(_wgrad_ws) >= 8:  # a backward uses a handful of shapes; keep the cache bounded
             _wgrad_ws.clear()
         _wgrad_ws[key] = ws
-    out = torch.empty(Ka, Kb, dtype=out_dtype, device=a.device)
+    wide = widen and out_dtype == BF16
+    out = torch.empty(Ka, Kb, dtype=torch.float32 if wide else out_dtype, device=a.device)
     call("vk_wgrad", ptr(a), a.stride(0), ptr(b), b.stride(0), N, Ka, Kb, ptr(out),
-         VK_DTYPE_BF16 if out_dtype == BF16 else VK_DTYPE_F32, ptr(ws), ws.numel(), stream_handle())
+         VK_DTYPE_F32_BF16 if wide else VK_DTYPE_BF16 if out_dtype == BF16 else VK_DTYPE_F32, ptr(ws), ws.numel(), stream_handle())
     return out
+
+
+def _weights_bf16(ws, outs, transpose):
+    n = len(ws)
+    P, I = ctypes.c_void_p * n, ctypes.c_int32 * n
+    call("vk_weights_bf16", P(*[w.data_ptr() for w in ws]), P(*[o.data_ptr() for o in outs]),
+         I(*[w.shape[0] for w in ws]), I(*[w.shape[1] for w in ws]), n, int(transpose), stream_handle())
+    return outs
+
+
+def _weights_ok(ws, dtype):
+    return bool(ws) and all(w.dim() == 2 and w.dtype == dtype and w.is_contiguous() and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0
+               and w.numel() and w.data_ptr() % 16 == 0 and w.device == ws[0].device for w in ws)
+
+
+def weights_bf16(ws):
+    """Each fp32 matrix of ws as a contiguous bf16 tensor (w.to(bfloat16)), in one launch; matrices that are not fp32,
+    contiguous and of multiples of 8 are cast by the tensor copy."""
+    for w in ws[:1]:
+        require_device(w, "weights_bf16")
+    if not _weights_ok(ws, torch.float32):
+        return [w.to(BF16).contiguous() for w in ws]
+    return _weights_bf16(ws, [torch.empty(w.shape, dtype=BF16, device=w.device) for w in ws], False)
+
+
+def weights_t(ws):
+    """Each bf16 matrix of ws transposed into a contiguous tensor (w.t().contiguous()), in one launch; matrices that are
+    not contiguous and of multiples of 8 by the tensor copy."""
+    for w in ws[:1]:
+        require_device(w, "weights_t")
+    if not _weights_ok(ws, BF16):
+        return [w.t().contiguous() for w in ws]
+    return _weights_bf16(ws, [torch.empty(w.shape[1], w.shape[0], dtype=BF16, device=w.device) for w in ws], True)
 
 
 def bias_act(y, bias, gelu):

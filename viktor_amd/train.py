@@ -98,12 +98,12 @@ class _Projector(torch.autograd.Function):
         x, pre, a, w2b = ctx.saved_tensors
         dy = dy.to(BF16).contiguous()
         gb2 = ops.act_backward(dy)
-        gw2 = ops.wgrad(dy, a)
+        gw2 = ops.wgrad(dy, a, widen=True)
         da = ops.linear(dy, w2b.t().contiguous())
         dz, gb1 = ops.act_backward(da, pre)
-        gw1 = ops.wgrad(dz, x)
+        gw1 = ops.wgrad(dz, x, widen=True)
         # autocast rounds the bias gradients to bf16 like the weight gradients
-        return None, gw1.float(), gb1.to(BF16).float(), gw2.float(), gb2.to(BF16).float()
+        return None, gw1, gb1.to(BF16).float(), gw2, gb2.to(BF16).float()
 
 
 class _LMHead(torch.autograd.Function):
@@ -176,8 +176,10 @@ class _DecoderStack(torch.autograd.Function):
         L = cfg.n_layers
         N = x.shape[0]
         norm_slot = {8 * i + _LAYER_PARAMS.index(n) for i in range(L) for n in _NORMS} | {8 * L}
-        w = [p.detach().float().contiguous() if j in norm_slot else p.detach().to(BF16).contiguous()
-             for j, p in enumerate(params)]
+        w = [p.detach().float().contiguous() if j in norm_slot else p.detach() for j, p in enumerate(params)]
+        mats = [j for j in range(len(params)) if j not in norm_slot]
+        for j, m in zip(mats, ops.weights_bf16([w[j] for j in mats])):
+            w[j] = m
         plan, rpos, cos, sin = meta["plan"], meta["rpos"], meta["cos"], meta["sin"]
         x = x.detach().float().contiguous()  # read only: every layer writes its stream into a new buffer
         h = ops.rmsnorm_f32(x, w[0], eps)
@@ -213,6 +215,7 @@ class _DecoderStack(torch.autograd.Function):
         x_final = ctx.x_final
         N, d = x_final.shape
         grads = [None] * len(w)
+        wt = ops.weights_t([w[8 * i + j] for i in range(L) for j in (1, 4, 6, 7)])  # Wqkv^T, Wo^T, Wgu^T, Wd^T per layer
         dh = torch.zeros(N, d, dtype=torch.float32, device=x_final.device)
         dh[meta["tok_rows"]] = dh_tok.float()
         # each norm backward also writes its fp32 input gradient rounded to bf16 (the next products' operand)
@@ -220,23 +223,24 @@ class _DecoderStack(torch.autograd.Function):
         dx, grads[8 * L] = ops.rmsnorm_backward(x_final, w[8 * L], dh, eps, dx_bf16=dxb)  # dx: d loss / d x_L (fp32)
         for i in reversed(range(L)):
             x_in, h, qkv, q, k, v, o, lse, x_mid, h2, gu, g = saved[i]
-            wa, wqkv, wqn, wkn, wo, wm, wgu, wd = w[8 * i:8 * i + 8]
+            wa, _, wqn, wkn, _, wm, _, _ = w[8 * i:8 * i + 8]
+            wqkv_t, wo_t, wgu_t, wd_t = wt[4 * i:4 * i + 4]
             # x_{i+1} = x_mid + g Wd^T
             dm = dxb
-            gd = ops.wgrad(dm, g)
-            dg = ops.linear(dm, wd.t().contiguous())
+            gd = ops.wgrad(dm, g, widen=True)
+            dg = ops.linear(dm, wd_t)
             dgu = ops.swiglu_backward(gu, dg)
-            ggu = ops.wgrad(dgu, h2)
-            dh2 = ops.linear(dgu, wgu.t().contiguous())
+            ggu = ops.wgrad(dgu, h2, widen=True)
+            dh2 = ops.linear(dgu, wgu_t)
             da = torch.empty(N, d, dtype=BF16, device=dx.device)
             dx, gm = ops.rmsnorm_backward(x_mid, wm, dh2, eps, dres=dx, dx_bf16=da)  # d / d x_mid
             # x_mid = x_in + o Wo^T
-            go = ops.wgrad(da, o.view(N, H * D))
-            do = ops.linear(da, wo.t().contiguous()).view(N, H, D)
+            go = ops.wgrad(da, o.view(N, H * D), widen=True)
+            do = ops.linear(da, wo_t).view(N, H, D)
             dq, dk, dv = ops.attention_backward(q, k, v, o, do, lse, plan.attn, plan.keys)
             dqkv, gqn, gkn = ops.qknorm_rope_backward(qkv, wqn, wkn, cos, sin, rpos, dq, dk, dv, eps, H, HKV, D)
-            gqkv = ops.wgrad(dqkv, h)
-            dhh = ops.linear(dqkv, wqkv.t().contiguous())
+            gqkv = ops.wgrad(dqkv, h, widen=True)
+            dhh = ops.linear(dqkv, wqkv_t)
             dxb = torch.empty(N, d, dtype=BF16, device=dx.device) if i > 0 else None
             dx, ga = ops.rmsnorm_backward(x_in, wa, dhh, eps, dres=dx, dx_bf16=dxb)  # d / d x_in
             grads[8 * i:8 * i + 8] = [ga, gqkv, gqn, gkn, go, gm, ggu, gd]
