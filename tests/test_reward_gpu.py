@@ -114,6 +114,20 @@ def test_strict_identity_at_the_edges_of_lanes_and_wavefronts(m):
     _check(calls, labels, scored, [i % 2 for i in range(len(calls))])
 
 
+@pytest.mark.parametrize("m", [3, 4, 5, 255, 256, 257, 767, 768, 769, 2049])
+def test_strict_identity_at_the_edges_of_column_blocks(m):
+    """Labels that end on or beside a lane's 4 rows and a wavefront's 256, calls that end on or beside the blocks of 64
+    columns whose steps run without the column test."""
+    rng = np.random.default_rng(m)
+    labels = ["".join(rng.choice(list("ACGT"), m)), "".join(rng.choice(list("AC"), max(1, m - 5)))]
+    scored = [rng.random(len(l)) > 0.3 for l in labels]
+    calls = ["".join(rng.choice(list("ACGT"), n)) for n in (127, 128, 191, 192, 193, 447, 448, 449)]
+    calls += [_mutate(rng, labels[0], 0.1), _mutate(rng, labels[1], 0.4)]
+    if m in (512, 4095):
+        calls.append("".join(rng.choice(list("ACGT"), 8192)))
+    _check(calls, labels, scored, [i % 2 for i in range(len(calls))])
+
+
 @pytest.mark.parametrize("k,T", [(1, 1), (1, 1023), (1, 1024), (1, 1025), (4, 3), (4, 2050)])
 def test_token_rows_at_the_edges_of_a_pass(k, T):
     """Rows that end on or beside a workgroup's pass of 1024 tokens, EOS at a pass's first and last token, ids outside

@@ -12,25 +12,29 @@
 // the traceback from the last cell with the same preference (no traceback pass, no per-cell storage). The
 // edit distance, and the count when every label base is scored, do not depend on the choice of path.
 //
-// MI355X design: the DP matrix as a systolic array. A wavefront owns 512 label rows, 8 consecutive ones per lane in
-// registers, and advances one call base per step: lane l is l columns behind lane 0, takes the row above its 8 (lane
-// l - 1's last row of the step before) and the call base through a one-lane DPP shift, and updates its 8 cells. Labels
-// past 512 bases take more wavefronts of the same workgroup, each 128 columns behind the one above it; the row between
+// MI355X design: the DP matrix as a systolic array. A wavefront owns 256 label rows, 4 consecutive ones per lane in
+// registers, and advances one call base per step: lane l is l columns behind lane 0, takes the row above its 4 (lane
+// l - 1's last row of the step before) and the call base through a one-lane DPP shift, and updates its 4 cells. Labels
+// past 256 bases take more wavefronts of the same workgroup, each 128 columns behind the one above it; the row between
 // two of them goes through a small LDS ring, handed over once per 64 columns at a barrier. A cell is one 32-bit word,
 //   distance << 18 | move << 16 | count,
 // so one v_min3_u32 over the three predecessors takes the smallest distance and, among equals, the preferred move
 // (0 diagonal, 1 deletion, 2 insertion) with the count that belongs to it; the move bits are then cleared.
-// Bound by the chain of about 7 integer instructions per cell, one wavefront per SIMD: 512 calls of about 850 bases
-// against labels of 700-1000 take 0.35 ms. The form before (a lane per cell of an anti-diagonal, three diagonals of
-// 16-bit pairs in LDS) took 5.17 ms: every step waited on its LDS reads and a barrier. (16 rows per lane in one
-// wavefront would double the steps' length on half the SIMDs; 4 rows would spend two thirds of a step on the shifts.)
+// Bound by the chain of integer instructions per cell. Steps whose 64 columns lie inside the call run without the
+// column test (its branch and the copies it forces), nine unrolled, and the last lane's row is collected by a lane
+// shift instead of a store per step; 4 rows per lane put two wavefronts on a SIMD where 8 left one. 512 calls of about
+// 850 bases against labels of 700-1000: 353 us with the test in every step and 8 rows per lane, 278 without it, 218
+// with 4 rows (labels of 510, one wavefront of 8 rows each: 6% slower with 4). The form before (a lane per cell of an
+// anti-diagonal, three diagonals of 16-bit pairs in LDS) took 5.17 ms: every step waited on its LDS reads and a barrier.
+#include <type_traits>
+
 #include "common.h"
 
 namespace vk {
 
-constexpr int RW_MAX_REF = 4096;   // label bases: 8 wavefronts of 512 rows
+constexpr int RW_MAX_REF = 4096;   // label bases: 16 wavefronts of 256 rows
 constexpr int RW_MAX_CALL = 8192;  // call bases: distances stay below 2^14, counts below 2^16
-constexpr int RW_R = 8;            // label rows per lane
+constexpr int RW_R = 4;            // label rows per lane
 constexpr int RW_ROWS = 64 * RW_R;
 constexpr uint32_t RW_ONE = 1u << 18, RW_DEL = 1u << 16, RW_INS = 2u << 16;
 
@@ -39,7 +43,12 @@ __device__ __forceinline__ uint32_t rw_shift(uint32_t v, uint32_t first) {
   return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(first), static_cast<int>(v), 0x138, 0xf, 0xf, false));
 }
 
-__global__ __launch_bounds__(512) void strict_identity_kernel(
+// q moved one lane down (lane l gets lane l + 1's), the last lane's v into lane 63
+__device__ __forceinline__ uint32_t rw_collect(uint32_t q, uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(q), 0x130, 0xf, 0xf, false));
+}
+
+__global__ __launch_bounds__(1024) void strict_identity_kernel(
     const uint8_t *__restrict__ calls, const int64_t *__restrict__ call_off, const int32_t *__restrict__ call_len,
     const uint8_t *__restrict__ refs, const int64_t *__restrict__ ref_off, const int32_t *__restrict__ ref_len,
     const uint8_t *__restrict__ scored, const int32_t *__restrict__ ref_of_call, int n_refs, int max_ref,
@@ -65,7 +74,7 @@ __global__ __launch_bounds__(512) void strict_identity_kernel(
   const uint8_t *rg = refs + ref_off[r], *sg = scored + ref_off[r], *cg = calls + call_off[c];
   const int waves = (m + RW_ROWS - 1) / RW_ROWS;  // wavefronts with rows of this label (<= the workgroup's)
 
-  // this lane's rows row0 + 1 .. row0 + 8 are label bases row0 .. row0 + 7 (rows past the label: never read by others)
+  // this lane's rows row0 + 1 .. row0 + 4 are label bases row0 .. row0 + 3 (rows past the label: never read by others)
   const int row0 = (wid * 64 + lane) * RW_R;
   uint32_t base[RW_R], cost[RW_R], left[RW_R];
   uint32_t own = 0;
@@ -96,17 +105,20 @@ __global__ __launch_bounds__(512) void strict_identity_kernel(
   // steps t = 1 .. n + 63 in blocks of 64: lane l updates column t - l. Wavefront w runs block p - 2 w in phase p: the
   // 64 columns it reads were finished, with their last lane's lag of 63, two blocks after they began
   const int blocks = n > 0 ? (n + 63 + 63) / 64 : 0;
-  uint32_t ch = 0;
+  uint32_t ch = 0, ring_out = 0;
   for (int p = 0; p < blocks + 2 * (waves - 1); ++p) {
     const int b = p - 2 * wid;
     if (wid < waves && b >= 0 && b < blocks) {
       const uint32_t next_ch = 64 * b + lane < n ? cg[64 * b + lane] : 0u;
       const uint32_t next_top = wid > 0 ? ring[wid - 1][b & 3][lane] : static_cast<uint32_t>(64 * b + lane + 1) * top_step;
-      for (int s = 0; s < 64; ++s) {
+      // a step; check: some lane may be outside columns 1 .. n (the first block, and those past column n - 64). The last
+      // lane's last row is collected in ring_out, the latest 64 steps' values in lane order: it lags 63 columns, so after
+      // step 62 they are the 64 columns of block b - 1
+      auto step = [&](auto check, int s) {
         const uint32_t top = rw_shift(left[RW_R - 1], __builtin_amdgcn_readlane(next_top, s));
         ch = rw_shift(ch, __builtin_amdgcn_readlane(next_ch, s));
         const int j = 64 * b + s + 1 - lane;
-        if (j >= 1 && j <= n) {
+        if (!check || (j >= 1 && j <= n)) {
           uint32_t d = diag, u = top;
 #pragma unroll
           for (int i = 0; i < RW_R; ++i) {
@@ -117,9 +129,29 @@ __global__ __launch_bounds__(512) void strict_identity_kernel(
             left[i] = u;
           }
           diag = top;
-          if (lane == 63 && wid + 1 < waves) ring[wid][((j - 1) >> 6) & 3][(j - 1) & 63] = u;
         }
+        ring_out = rw_collect(ring_out, left[RW_R - 1]);
+      };
+      constexpr std::true_type checked{};
+      constexpr std::false_type unchecked{};
+      const bool inside = b > 0 && 64 * (b + 1) <= n;
+      if (inside) {
+#pragma unroll 1
+        for (int s = 0; s < 63; s += 9) {
+#pragma unroll
+          for (int e = 0; e < 9; ++e) step(unchecked, s + e);
+        }
+      } else {
+#pragma unroll 1
+        for (int s = 0; s < 63; ++s) step(checked, s);
       }
+      if (wid + 1 < waves) ring[wid][(b - 1) & 3][lane] = ring_out;  // block b - 1 is complete
+      if (inside)
+        step(unchecked, 63);
+      else
+        step(checked, 63);
+      // the last block's first column is the last one anybody needs (64 blocks >= n + 63)
+      if (wid + 1 < waves && b == blocks - 1 && lane == 63) ring[wid][b & 3][0] = left[RW_R - 1];
     }
     if (waves > 1) __syncthreads();
   }
