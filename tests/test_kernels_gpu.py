@@ -675,10 +675,12 @@ def test_greedy_update_reference_signature():
 
 
 @pytest.mark.parametrize("T", [1, 255, 256, 257, 1024, 1025])
-@pytest.mark.parametrize("V,dtype", [(1, torch.float32), (7, BF), (8, torch.float32), (9, BF)])
+@pytest.mark.parametrize("V,dtype", [(1, torch.float32), (7, BF), (8, torch.float32), (9, BF), (32, torch.float32), (33, BF),
+                                     (343, torch.float32), (512, BF), (513, torch.float32)])
 def test_gspo_score_few_logits(V, T, dtype):
-    """The kernel that keeps a row's logits in registers, at the edges of its rounds and of its range (T = 1025 and V = 9
-    run the one that reads them twice), against fp64: 1e-5 for fp32 exponentials and sums of T terms."""
+    """A workgroup per sequence with its logits in registers (V <= 8, T <= 1024), a token per thread (T = 1025, V = 9, 32)
+    and a token per wavefront, in registers (33, 343, 512) or read again (513), at the edges of their rounds, against
+    fp64: 1e-5 for fp32 exponentials and sums of T terms."""
     g = gen(T + V)
     B = 3
     z = to_dev(torch.randn(B, T, V, generator=g), dtype)

@@ -8,8 +8,7 @@
 //   dL/dz[b,t,v] = (1/N) g_b s_b mask[b,t] / n_bases[b] (onehot(y)[v] - softmax(z[b,t])[v]),
 //   g_b = d pg_b / d s_b, with torch.minimum splitting ties evenly and clamp passing its gradient on
 //   the closed interval.
-// One workgroup per sequence; tokens are spread over threads (small vocabularies) or wavefronts
-// (large ones); every reduction runs in a fixed order, so results are bitwise reproducible.
+// Every reduction runs in a fixed order, so results are bitwise reproducible.
 #include <math.h>
 
 #include "common.h"
@@ -57,15 +56,13 @@ __device__ __forceinline__ float block_sum(float v, float *scratch) {
   return t;
 }
 
-// From the masked sum of a sequence: its ratio and objective, and (returned) the factor of its logits' gradient.
-__device__ __forceinline__ float ratio_terms(float tot, float nb, float A, float eps_lo, float eps_hi, float inv_n,
-                                             float *s_out, float *pg_out) {
-  const float s = expf(tot / nb);
+// From a sequence's ratio: its objective, and (returned) the factor of its logits' gradient.
+__device__ __forceinline__ float ratio_terms(float s, float nb, float A, float eps_lo, float eps_hi, float inv_n,
+                                             float &pg) {
   const float lo = 1.0f - eps_lo, hi = 1.0f + eps_hi;
   const float sc = fminf(fmaxf(s, lo), hi);
   const float a1 = s * A, a2 = sc * A;
-  *s_out = s;
-  *pg_out = -fminf(a1, a2);
+  pg = -fminf(a1, a2);
   // d min(a1, a2) / ds: a1 branch slope A, a2 branch slope A * [lo <= s <= hi]; ties split evenly
   const float d2 = (s >= lo && s <= hi) ? A : 0.f;
   float dmin;
@@ -134,7 +131,13 @@ __global__ __launch_bounds__(GS_THREADS) void gspo_score_few_kernel(
   }
   if (!ratio) return;
   const float tot = block_sum(part, scratch);
-  if (tid == 0) coef_sh = ratio_terms(tot, n_bases[b], adv[b], eps_lo, eps_hi, inv_n, s_out + b, pg_out + b);
+  if (tid == 0) {
+    const float nb = n_bases[b], sr = expf(tot / nb);
+    float pg;
+    coef_sh = ratio_terms(sr, nb, adv[b], eps_lo, eps_hi, inv_n, pg);
+    s_out[b] = sr;
+    pg_out[b] = pg;
+  }
   if (dlogits == nullptr) return;
   __syncthreads();
   const float coef = coef_sh;
@@ -156,63 +159,154 @@ __global__ __launch_bounds__(GS_THREADS) void gspo_score_few_kernel(
   }
 }
 
+// Larger vocabularies or longer rows: a token per wavefront (V > 32; GS_TW tokens of a wavefront at once) or per thread,
+// over the whole batch. (A workgroup per sequence, its four wavefronts taking every fourth token twice, left most CUs
+// idle and waited for each token's round trips. Loss and gradient of 64 x 1024 tokens of 343 bf16 logits: 2176 -> 135
+// us, of them 90 in these three kernels; of 8 x 512: 674 -> 98.) A token's logits stay in registers (V <= 64 GS_VR)
+// between its max, sum and gradient.
+constexpr int GS_VR = 8, GS_TW = 2;
+
+// z[k] = logit lane + 64 k of a row (-inf past V), its max and log-sum-exp
+template <bool BF16>
+__device__ __forceinline__ void row_regs(const void *lg, int64_t base, int V, int lane, float (&z)[GS_VR]) {
+#pragma unroll
+  for (int k = 0; k < GS_VR; ++k) z[k] = lane + 64 * k < V ? logit_at<BF16>(lg, base + lane + 64 * k) : -INFINITY;
+}
+__device__ __forceinline__ float lse_regs(const float (&z)[GS_VR], int V, int lane) {
+  float mx = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < GS_VR; ++k) mx = fmaxf(mx, z[k]);
+  mx = wave_max(mx);
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < GS_VR; ++k)
+    if (lane + 64 * k < V) s += expf(z[k] - mx);
+  return mx + logf(wave_sum(s));
+}
+
 template <bool BF16, bool WAVE_PER_TOKEN>
-__global__ __launch_bounds__(GS_THREADS) void gspo_score_kernel(
-    const void *__restrict__ logits, const int64_t *__restrict__ targets, const uint8_t *__restrict__ mask,
-    const float *__restrict__ old_lp, const float *__restrict__ n_bases, const float *__restrict__ adv, float eps_lo,
-    float eps_hi, float inv_n, float *__restrict__ lp_out, float *__restrict__ s_out, float *__restrict__ pg_out,
-    float *__restrict__ dlogits, int64_t T, int V) {
-  __shared__ float scratch[GS_THREADS / 64];
-  __shared__ float coef_sh;
-  const int64_t b = blockIdx.x;
+__global__ __launch_bounds__(GS_THREADS) void gspo_lp_kernel(const void *__restrict__ logits,
+                                                            const int64_t *__restrict__ targets,
+                                                            float *__restrict__ lp_out, int64_t n, int V) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int stride = WAVE_PER_TOKEN ? GS_THREADS / 64 : GS_THREADS;
-  const int first = WAVE_PER_TOKEN ? wid : tid;
-  const bool ratio = old_lp != nullptr && adv != nullptr && n_bases != nullptr;
-
-  // pass 1: lp and the masked sum of (lp - old)
-  float part = 0.f;
-  for (int64_t t = first; t < T; t += stride) {
-    const int64_t row = b * T + t;
-    int64_t y = targets[row];
-    y = (y < 0 || y >= V) ? 0 : y;
+  auto target = [&](int64_t row) {
+    const int64_t y = targets[row];
+    return (y < 0 || y >= V) ? int64_t(0) : y;
+  };
+  if (!WAVE_PER_TOKEN) {
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * GS_THREADS + tid;
+    if (row >= n) return;
     float mx, lse;
-    if (WAVE_PER_TOKEN)
-      lse_wave<BF16>(logits, row * V, V, lane, mx, lse);
-    else
-      lse_thread<BF16>(logits, row * V, V, mx, lse);
-    const float lp = logit_at<BF16>(logits, row * V + y) - lse;
-    if (!WAVE_PER_TOKEN || lane == 0) {
-      lp_out[row] = lp;
-      if (ratio && mask[row]) part += lp - old_lp[row];
-    }
+    lse_thread<BF16>(logits, row * V, V, mx, lse);
+    lp_out[row] = logit_at<BF16>(logits, row * V + target(row)) - lse;
+    return;
   }
-  if (!ratio) return;
-  const float tot = block_sum(part, scratch);
-  if (tid == 0) coef_sh = ratio_terms(tot, n_bases[b], adv[b], eps_lo, eps_hi, inv_n, s_out + b, pg_out + b);
-  if (dlogits == nullptr) return;
-  __syncthreads();
-  const float coef = coef_sh;
+  const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * (GS_THREADS / 64) + wid) * GS_TW;
+  if (V > 64 * GS_VR) {
+    for (int i = 0; i < GS_TW && r0 + i < n; ++i) {
+      float mx, lse;
+      lse_wave<BF16>(logits, (r0 + i) * V, V, lane, mx, lse);
+      if (lane == 0) lp_out[r0 + i] = logit_at<BF16>(logits, (r0 + i) * V + target(r0 + i)) - lse;
+    }
+    return;
+  }
+  float z[GS_TW][GS_VR], zy[GS_TW];
+#pragma unroll
+  for (int i = 0; i < GS_TW; ++i) {
+    const int64_t row = min(r0 + i, n - 1);
+    row_regs<BF16>(logits, row * V, V, lane, z[i]);
+    zy[i] = logit_at<BF16>(logits, row * V + target(row));
+  }
+#pragma unroll
+  for (int i = 0; i < GS_TW; ++i) {
+    const float lse = lse_regs(z[i], V, lane);
+    if (lane == 0 && r0 + i < n) lp_out[r0 + i] = zy[i] - lse;
+  }
+}
 
-  // pass 2: dL/dz = coef * mask * (onehot - softmax)
-  for (int64_t t = first; t < T; t += stride) {
-    const int64_t row = b * T + t;
-    const float c = mask[row] ? coef : 0.f;
-    int64_t y = targets[row];
-    y = (y < 0 || y >= V) ? 0 : y;
+// A workgroup per sequence: the masked sum of (lp - old), the ratio and the objective.
+__global__ __launch_bounds__(GS_THREADS) void gspo_ratio_kernel(const float *__restrict__ lp, const uint8_t *__restrict__ mask,
+                                                               const float *__restrict__ old_lp,
+                                                               const float *__restrict__ n_bases,
+                                                               const float *__restrict__ adv, float eps_lo, float eps_hi,
+                                                               float inv_n, float *__restrict__ s_out,
+                                                               float *__restrict__ pg_out, int64_t T) {
+  __shared__ float scratch[GS_THREADS / 64];
+  const int64_t b = blockIdx.x;
+  float part = 0.f;
+  for (int64_t t = threadIdx.x; t < T; t += GS_THREADS)
+    if (mask[b * T + t]) part += lp[b * T + t] - old_lp[b * T + t];
+  const float tot = block_sum(part, scratch);
+  if (threadIdx.x == 0) {
+    const float nb = n_bases[b], s = expf(tot / nb);
+    float pg;
+    ratio_terms(s, nb, adv[b], eps_lo, eps_hi, inv_n, pg);
+    s_out[b] = s;
+    pg_out[b] = pg;
+  }
+}
+
+// dL/dz = coef * mask * (onehot - softmax)
+template <bool BF16, bool WAVE_PER_TOKEN>
+__global__ __launch_bounds__(GS_THREADS) void gspo_grad_kernel(const void *__restrict__ logits,
+                                                              const int64_t *__restrict__ targets,
+                                                              const uint8_t *__restrict__ mask,
+                                                              const float *__restrict__ s_in,
+                                                              const float *__restrict__ n_bases,
+                                                              const float *__restrict__ adv, float eps_lo, float eps_hi,
+                                                              float inv_n, float *__restrict__ dlogits, int64_t n,
+                                                              int64_t T, int V) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  auto factor = [&](int64_t row) {
+    if (!mask[row]) return 0.f;
+    const int64_t b = row / T;
+    float pg;
+    return ratio_terms(s_in[b], n_bases[b], adv[b], eps_lo, eps_hi, inv_n, pg);
+  };
+  auto target = [&](int64_t row) {
+    const int64_t y = targets[row];
+    return (y < 0 || y >= V) ? int64_t(0) : y;
+  };
+  if (!WAVE_PER_TOKEN) {
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * GS_THREADS + tid;
+    if (row >= n) return;
+    const float c = factor(row);
+    const int64_t y = target(row);
     float mx, lse;
-    if (WAVE_PER_TOKEN) {
+    lse_thread<BF16>(logits, row * V, V, mx, lse);
+    for (int v = 0; v < V; ++v)
+      dlogits[row * V + v] = c * ((v == y ? 1.f : 0.f) - expf(logit_at<BF16>(logits, row * V + v) - lse));
+    return;
+  }
+  const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * (GS_THREADS / 64) + wid) * GS_TW;
+  if (V > 64 * GS_VR) {
+    for (int i = 0; i < GS_TW && r0 + i < n; ++i) {
+      const int64_t row = r0 + i, y = target(row);
+      const float c = factor(row);
+      float mx, lse;
       lse_wave<BF16>(logits, row * V, V, lane, mx, lse);
-      for (int v = lane; v < V; v += 64) {
-        const float sm = expf(logit_at<BF16>(logits, row * V + v) - lse);
-        dlogits[row * V + v] = c * ((v == y ? 1.f : 0.f) - sm);
-      }
-    } else {
-      lse_thread<BF16>(logits, row * V, V, mx, lse);
-      for (int v = 0; v < V; ++v) {
-        const float sm = expf(logit_at<BF16>(logits, row * V + v) - lse);
-        dlogits[row * V + v] = c * ((v == y ? 1.f : 0.f) - sm);
-      }
+      for (int v = lane; v < V; v += 64)
+        dlogits[row * V + v] = c * ((v == y ? 1.f : 0.f) - expf(logit_at<BF16>(logits, row * V + v) - lse));
+    }
+    return;
+  }
+  float z[GS_TW][GS_VR], c[GS_TW];
+  int64_t y[GS_TW];
+#pragma unroll
+  for (int i = 0; i < GS_TW; ++i) {
+    const int64_t row = min(r0 + i, n - 1);
+    row_regs<BF16>(logits, row * V, V, lane, z[i]);
+    y[i] = target(row);
+    c[i] = factor(row);
+  }
+#pragma unroll
+  for (int i = 0; i < GS_TW; ++i) {
+    const float lse = lse_regs(z[i], V, lane);
+    if (r0 + i >= n) break;
+#pragma unroll
+    for (int k = 0; k < GS_VR; ++k) {
+      const int v = lane + 64 * k;
+      if (v < V) dlogits[(r0 + i) * V + v] = c[i] * ((v == y[i] ? 1.f : 0.f) - expf(z[i][k] - lse));
     }
   }
 }
@@ -262,27 +356,32 @@ extern "C" int vk_gspo_score(const void *logits, int32_t logits_dtype, const int
   hipStream_t st = VK_STREAM(stream);
   const bool wave = V > 32;
   const dim3 grid(static_cast<unsigned>(B));
-#define VK_GSPO_LAUNCH(BF, WV)                                                                                    \
-  gspo_score_kernel<BF, WV><<<grid, GS_THREADS, 0, st>>>(logits, targets, mask, ratio ? old_lp : nullptr, n_bases, \
-                                                         ratio ? adv : nullptr, eps_lo, eps_hi, inv_n, lp, s, pg,   \
-                                                         dlogits, T, V)
   // few logits per token and rows short enough to stay in registers; longer rows read their logits twice
   if (V <= GS_V && T <= GS_THREADS * GS_TPT) {
     auto kern = logits_dtype == VK_DTYPE_BF16 ? gspo_score_few_kernel<true> : gspo_score_few_kernel<false>;
     kern<<<grid, GS_THREADS, 0, st>>>(logits, targets, mask, ratio ? old_lp : nullptr, n_bases, ratio ? adv : nullptr,
                                       eps_lo, eps_hi, inv_n, lp, s, pg, dlogits, static_cast<int>(T), V);
-  } else if (logits_dtype == VK_DTYPE_BF16) {
-    if (wave)
-      VK_GSPO_LAUNCH(true, true);
-    else
-      VK_GSPO_LAUNCH(true, false);
   } else {
-    if (wave)
-      VK_GSPO_LAUNCH(false, true);
-    else
-      VK_GSPO_LAUNCH(false, false);
+    const bool bf = logits_dtype == VK_DTYPE_BF16;
+    const int64_t n = B * T, per = wave ? GS_THREADS / 64 * GS_TW : GS_THREADS, blocks = (n + per - 1) / per;
+    VK_CHECK_ARG(blocks < (int64_t(1) << 31), "gspo_score: too many tokens");
+    auto lpk = bf ? (wave ? gspo_lp_kernel<true, true> : gspo_lp_kernel<true, false>)
+                  : (wave ? gspo_lp_kernel<false, true> : gspo_lp_kernel<false, false>);
+    lpk<<<static_cast<unsigned>(blocks), GS_THREADS, 0, st>>>(logits, targets, lp, n, V);
+    if (ratio) {
+      int rc = launch_status("gspo_score log-probs");
+      if (rc != VK_OK) return rc;
+      gspo_ratio_kernel<<<grid, GS_THREADS, 0, st>>>(lp, mask, old_lp, n_bases, adv, eps_lo, eps_hi, inv_n, s, pg, T);
+      rc = launch_status("gspo_score ratio");
+      if (rc != VK_OK) return rc;
+    }
+    if (ratio && dlogits != nullptr) {
+      auto gk = bf ? (wave ? gspo_grad_kernel<true, true> : gspo_grad_kernel<true, false>)
+                   : (wave ? gspo_grad_kernel<false, true> : gspo_grad_kernel<false, false>);
+      gk<<<static_cast<unsigned>(blocks), GS_THREADS, 0, st>>>(logits, targets, mask, s, n_bases, adv, eps_lo, eps_hi,
+                                                              inv_n, dlogits, n, T, V);
+    }
   }
-#undef VK_GSPO_LAUNCH
   int rc = launch_status("gspo_score");
   if (rc != VK_OK || !ratio) return rc;
   gspo_loss_kernel<<<1, GS_THREADS, 0, st>>>(pg, B, inv_n, loss);
