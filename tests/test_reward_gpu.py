@@ -102,7 +102,7 @@ def test_rewards_from_tokens_equal_rewards_from_strings():
 
 @pytest.mark.parametrize("m", [1, 7, 8, 9, 511, 512, 513, 1023, 1024, 1025, 2500, 4095])
 def test_strict_identity_at_the_edges_of_lanes_and_wavefronts(m):
-    """Labels that end on or beside a lane's 8 rows and a wavefront's 512, calls beside a block of 64 columns, up to the
+    """Labels that end on or beside multiples of a lane's rows and of a wavefront's, calls beside a block of 64 columns, up to the
     longest of both."""
     rng = np.random.default_rng(m)
     labels = ["".join(rng.choice(list("ACGT"), m)), "".join(rng.choice(list("AC"), max(1, m - 5)))]
