@@ -173,6 +173,29 @@ def test_linear_large_m_slab_counts(M, K):
         assert torch.equal(ops.linear_residual_big(x, wr, r), ss) and torch.equal(r, new)
 
 
+@pytest.mark.parametrize("M", [1, 63, 65, 129, 1000, 4100])
+def test_small_batch_tiles_same_bits(M):
+    """Batches too small for 128 x 128 tiles on every CU run 64 x 64 and 64 x 128 tiles: every epilogue's rows have the
+    bits of the same rows inside a batch that runs 128 x 128 ones (odd slab count, ragged columns)."""
+    from viktor_amd._lib import call, ptr, stream_handle
+    g = gen(M)
+    big_m, K, N = 20000, 192, 328
+    xb = to_dev(R.bf(torch.randn(big_m, K, generator=g)), BF)
+    w = to_dev(R.bf(torch.randn(2 * N, K, generator=g) / math.sqrt(K)), BF)
+    x = xb[7:7 + M].contiguous()
+    for epi, dt in ((0, BF), (1, torch.float32), (2, BF)):
+        out = [torch.empty(t.shape[0], N, dtype=dt, device=DEV) for t in (x, xb)]
+        for t, o in zip((x, xb), out):
+            call("vk_gemm_rows", ptr(t), ptr(w), ptr(o), t.shape[0], N, K, epi, stream_handle())
+        assert torch.equal(out[0], out[1][7:7 + M])
+    wr = w[:512].contiguous()
+    for dt in (BF, torch.float32):
+        rb = to_dev(torch.randn(big_m, 512, generator=g), dt)
+        r = rb[7:7 + M].clone()
+        ss, ssb = ops.linear_residual_big(x, wr, r), ops.linear_residual_big(xb, wr, rb)
+        assert torch.equal(r, rb[7:7 + M]) and torch.equal(ss, ssb[7:7 + M])
+
+
 def test_linear_wide_tiles_same_bits():
     """256 row blocks of 256 fill the chip with 256 x 256 tiles at K >= 1024; a row's bits are those of the 128 x 128
     tiles that a smaller batch runs."""

@@ -3,7 +3,7 @@
 // MI355X design (M = tokens or frames x N = 512..4096 x K = 512..3072):
 //   * 128 x 128 output tile per workgroup of 4 wavefronts, each 64 x 64 (16 fp32 MFMA tiles, 64 accumulator
 //     registers), two workgroups per CU: one workgroup's barriers and epilogue overlap the other's MFMAs, and a
-//     packed batch of a few thousand rows still fills the chip.
+//     packed batch of a few thousand rows still fills the chip (smaller ones take 64 x 128 and 64 x 64 tiles).
 //   * What bounds the K loop: with the MFMAs and LDS reads alone it runs at 1820 TFLOP/s (MFMAs alone 2080), with the
 //     loads alone at the rate of the global->LDS stream. That stream is issued as direct loads (buffer_load .. lds,
 //     16 bytes a lane, no registers) of 64-wide K slabs: 8 lanes take a row's whole 128-byte line, 24-29 TB/s over
@@ -46,10 +46,12 @@ struct GbShape {
   static constexpr int XLOADS = BM / RPL / WAVES;                      // x instructions per wave per stage
   static constexpr int WLOADS = BW / RPL / WAVES;
   static constexpr int LOADS = XLOADS + WLOADS;
-  static constexpr int WG_PER_CU = SMEM > 81920 ? 1 : 2;
-  static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4;
+  static constexpr int WG_PER_CU = SMEM > 81920 ? 1 : SMEM > 53248 ? 2 : 3;
+  static constexpr int WAVES_PER_SIMD = WG_PER_CU * WAVES / 4 > 0 ? WG_PER_CU * WAVES / 4 : 1;
 };
 using GbWide = GbShape<2, 4, 8>;    // 256 x 256, 128 KB: one workgroup of 8 wavefronts per CU
+using GbFlat = GbShape<2, 2, 2>;    // 64 x 128, 48 KB: up to three workgroups per CU
+using GbSmall = GbShape<2, 1, 2>;   // 64 x 64, 32 KB, two wavefronts
 using GbSquare = GbShape<2, 2, 4>;  // 128 x 128, 64 KB: two workgroups per CU
 
 typedef __attribute__((address_space(3))) void lds_void;
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(64 * SH::WAVES, SH::WAVES_PER_SIMD) void gemm_big_k
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   bf16x8 xa[FX], wa[4], xb[FX], wb[4];
-  if (FX == 4) read_frags(first, 0, xa, wa);
+  if (FX != 8) read_frags(first, 0, xa, wa);
   // The residual epilogues' operands (old rows, bias) are loaded in the last slab but one, behind the last direct loads,
   // so their round trips pass under its MFMAs (M = 131136, N = 512: 115 -> 111 us at K = 512, 290 -> 269 at K = 1536).
   // The QKV epilogues' (QK-norm weights, every row's rotary position; the table rows, which depend on the positions,
@@ -637,6 +639,20 @@ static int launch_big(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int 
     const int64_t tiles = (M + GbWide::BM - 1) / GbWide::BM * ((N + GbWide::BW - 1) / GbWide::BW);
     const int64_t cus = device_cus_cached(), rounds = (tiles + cus - 1) / cus;
     if (K >= 1024 && 8 * tiles >= 7 * rounds * cus) return launch_big_shape<EPI, GbWide>(x, w, y, M, N, K, qa, s);
+  }
+  // Batches whose 128 x 128 tiles leave CUs without one take smaller tiles (the same bits): a tile is a chain of slabs,
+  // and more, shorter chains run side by side. Residual product N = 512, K = 512 / 1536 / 2048, us with 128 x 128, 64 x
+  // 128, 64 x 64 tiles: M = 1324 (44 tiles of 128 x 128) 9.3 / 15.7 / 22.6, 8.1 / 10.5 / 18.6, 8.3 / 9.3 / 10.9; 4099
+  // (132) 9.7 / 21.1 / 24.3, 8.5 / 17.0 / 21.4, 8.6 / 17.4 / 21.7; 7500 (236) 10.0 / 21.4 / 25.6, 9.3 / 18.8 / 22.8,
+  // 10.6 / 21.1 / 25.6; 9000 (284) 13.7 / 25.4 / 29.4, 11.9 / 26.6 / 30.6, 13.5 / 31.3 / 38.8. The Wqkv epilogues keep
+  // one shape: the compiler contracts their fp32 rotation differently in another, and a row's bits are not to depend on
+  // the batch.
+  if constexpr (EPI != GB_QKV && EPI != GB_QKV_BF16 && EPI != GB_QKV_W32) {
+    constexpr int OUT_COLS = EPI == GB_SWIGLU ? GbSquare::BW / 2 : GbSquare::BW;
+    const int64_t tiles = (M + GbSquare::BM - 1) / GbSquare::BM * ((N + OUT_COLS - 1) / OUT_COLS);
+    const int64_t cus = device_cus_cached();
+    if (2 * tiles <= cus) return launch_big_shape<EPI, GbSmall>(x, w, y, M, N, K, qa, s);
+    if (tiles <= cus) return launch_big_shape<EPI, GbFlat>(x, w, y, M, N, K, qa, s);
   }
   return launch_big_shape<EPI, GbSquare>(x, w, y, M, N, K, qa, s);
 }
