@@ -1096,11 +1096,10 @@ def test_norm_linear(M, mode):
     assert ok, err
 
 
-@pytest.mark.parametrize("M", [1, 15, 16, 17, 31, 32, 33])
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 15, 16, 17, 31, 32, 33])
 def test_few_row_products(M):
-    """The products of at most 16 (o + residual) / 32 (gate_up + SwiGLU) rows at the edges of their row blocks, with a
-    ragged count of column blocks: the oracle's rounding points, rows past M untouched, the same bits for a row of a
-    larger call that runs the same kernel."""
+    """The products of at most 8 (o + residual) / 32 (gate_up + SwiGLU) rows at the edges of their row blocks, with a
+    ragged count of column blocks: the oracle's rounding points, rows past M untouched, the same bits for a row alone."""
     g = gen(M + 5)
     K = 512
     a = R.bf(torch.randn(M, K, generator=g))
@@ -1121,7 +1120,32 @@ def test_few_row_products(M):
     assert ok, err
     one = ops.norm_linear(to_dev(r[:1].contiguous(), BF), to_dev(nw, BF), 1e-6, to_dev(wg, BF), swiglu=True,
                           ss=to_dev(_row_ss(r[:1])))
-    assert M > 32 or torch.equal(one[0], out[0])
+    assert torch.equal(one[0], out[0])
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33])
+def test_decode_product_bits_do_not_depend_on_the_batch(M):
+    """o + residual with its row sums of squares, and gate_up + SwiGLU from such sums: the first M rows of a batch of 512
+    (the decode step's tiles) and of 40 alone have the same bits, N = 512 / 1536 and narrower ones."""
+    g = gen(M + 50)
+    K = 512
+    a, x, r = (to_dev(R.bf(torch.randn(512, K, generator=g)), BF) for _ in range(3))
+    nw = to_dev(R.bf(torch.rand(K, generator=g) + 0.5), BF)
+    ss = to_dev(_row_ss(r.float().cpu()))
+    for N in (512, 96):
+        w = to_dev(R.bf(torch.randn(N, K, generator=g) / math.sqrt(K)), BF)
+        got = []
+        for rows in (M, 40, 512):
+            y = x[:rows, :N].contiguous().clone()
+            sums = torch.empty(rows, 16, device=DEV) if N == 512 else None
+            ops.linear_residual(a[:rows], w, y, ss_out=sums)
+            got.append((y[:M], None if sums is None else sums[:M]))
+        for y, sums in got[1:]:
+            assert torch.equal(got[0][0], y) and (sums is None or torch.equal(got[0][1], sums))
+    for N in (1536, 96, 48):
+        w = to_dev(R.bf(torch.randn(2 * N, K, generator=g) / math.sqrt(K)), BF)
+        got = [ops.norm_linear(r[:rows], nw, 1e-6, w, swiglu=True, ss=ss[:rows])[:M] for rows in (M, 40, 512)]
+        assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
 @pytest.mark.parametrize("B,S", [(1, 33), (1, 17 * 256 + 5), (2, 70 * 256 + 31), (3, 512)])

@@ -1332,35 +1332,41 @@ static int launch_panel(const SkinnyArgs &a, hipStream_t s) {
 
 // ---- products of a few rows (a decode step of at most FR_ROWS sequences) at K = 512 -----------------------
 //
-// With so few rows a product is one round trip to the weights and back: the kernel is that, and nothing in series
-// with it. 8 wavefronts split K; each loads its share of the weight rows (16 per block) and of x straight into MFMA
-// fragments, everything issued before the first wait (the LDS rings above bring K in stages, several round trips
-// and their barriers), the row norm is applied to the x fragment in registers, and the wavefronts' fp32 tiles meet in
-// LDS, summed in wavefront order. EPI_RESID: 32 output columns per workgroup; EPI_SWIGLU: 16 (and their up rows).
-// XB blocks of 16 rows. In a replayed graph, us per product (4 / 16 / 32 rows): gate_up + SwiGLU 6.4 / 6.4 / 6.6 ->
-// 3.2 / 3.6 / 4.6; o + residual 3.6 / 3.7 / 3.8 -> 3.2 / 3.5 / 4.3, so the latter only up to 16 rows. The same form
-// for the down product (K = 1536: 16 workgroups of 96 KB of weights) and for qkv (12 of 64 KB) measured 5.9 against
-// 5.8 and 6.0 against 5.5 us in the step, bound by what one CU pulls, and is not used.
-constexpr int FR_WAVES = 8, FR_STEPS = 2, FR_K = 32 * FR_STEPS * FR_WAVES;
-constexpr int FR_ROWS = 32;
+// With so few rows a product is one round trip to the weights and back: the kernel is that, and little in series with
+// it. 8 wavefronts load two K steps each of the weight rows (2 blocks of 16) and of x straight into MFMA fragments,
+// everything issued before the first wait (the LDS rings above bring K in stages, several round trips and their
+// barriers), apply the row norm to the x fragments in registers and lay all fragments out in LDS. K is then added in the
+// order of the kernels that take more rows, so a row's bits do not depend on how many are beside it: EPI_SWIGLU (16
+// output columns and their up rows per workgroup) one chain of 16 MFMAs per block, EPI_RESID (32 output columns) two
+// halves of 8 and their sum, a wavefront per chain. XB blocks of 16 rows. In a replayed graph, us per product (1 / 4 / 8
+// / 16 / 32 rows): gate_up + SwiGLU 6.3 / 6.3 / 6.4 / 6.5 / 6.7 -> 3.2 / 3.4 / 3.6 / 3.8 / 5.0; o + residual 3.6 / 3.7 /
+// 3.6 / 3.7 / - -> 3.4 / 3.5 / 3.6 / 3.8 / -, so the latter only up to 8 rows. (With each wavefront's two steps summed
+// by themselves and the 8 partial tiles in LDS it was 0.1-0.2 us faster, but in an order of K of its own.) The down
+// product (K = 1536: 16 workgroups of 96 KB of weights) and qkv (12 of 64 KB) are bound by what one CU pulls and gain
+// nothing from it.
+constexpr int FR_WAVES = 8, FR_STEPS = 2, FR_KSTEPS = FR_WAVES * FR_STEPS, FR_K = 32 * FR_KSTEPS;
+constexpr int FR_ROWS = 32, FR_RES_ROWS = 8;
 static_assert(FR_K == PG_NORM_K && PG_SS_COLS == 32, "the row sums of squares are one per 32 columns of 512");
 
 template <int EPI, int XB>
 __global__ __launch_bounds__(64 * FR_WAVES) void few_rows_kernel(const SkinnyArgs p) {
   constexpr bool SWI = EPI == EPI_SWIGLU;  // with the row norm; EPI_RESID without
+  static_assert(SWI || XB == 1, "the residual epilogue has a thread per output of 16 rows");
+  constexpr int PARTS = SWI ? 1 : 2;  // chains K is split into
   constexpr int PITCH = 32 + 4;
-  __shared__ __attribute__((aligned(16))) float part[FR_WAVES * XB * 16 * PITCH];
+  __shared__ __attribute__((aligned(16))) u32x4 frag[2 + XB][FR_KSTEPS][64];  // two blocks of w, the blocks of x
+  __shared__ __attribute__((aligned(16))) float part[PARTS][XB * 16 * PITCH];
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fg = lane >> 4;
   const int k0 = wid * 32 * FR_STEPS + 8 * fg;
   const int M = static_cast<int>(p.M);
   const int n0 = blockIdx.x * (SWI ? 16 : 32);
-  // this thread's outputs: rows er + 16 t, t < XB, at column ec (EPI_SWIGLU: threads 0 .. 255)
-  const int er = SWI ? tid >> 4 & 15 : tid >> 5, ec = SWI ? tid & 15 : tid & 31;
+  const int row = SWI ? tid >> 4 : tid >> 5, col = SWI ? tid & 15 : tid & 31;  // this thread's output
+  bf16_t *const dst = static_cast<bf16_t *>(p.y) + static_cast<int64_t>(min(row, M - 1)) * p.N + n0 + col;
 
   u32x4 xf[XB][FR_STEPS], nw[SWI ? FR_STEPS : 1], wf[2][FR_STEPS];
   f32x4 sq[XB][SWI ? 4 : 1];
-  bf16_t old[XB];
+  bf16_t old = 0;
 #pragma unroll
   for (int t = 0; t < XB; ++t) {
     const int64_t r = min(16 * t + fr, M - 1);
@@ -1377,19 +1383,15 @@ __global__ __launch_bounds__(64 * FR_WAVES) void few_rows_kernel(const SkinnyArg
   }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int64_t row = (SWI ? j * p.N + n0 : n0 + 16 * j) + fr;
+    const int64_t wr = (SWI ? static_cast<int64_t>(j) * p.N + n0 : n0 + 16 * j) + fr;
 #pragma unroll
-    for (int s = 0; s < FR_STEPS; ++s) wf[j][s] = *reinterpret_cast<const u32x4 *>(p.w + row * FR_K + k0 + 32 * s);
+    for (int s = 0; s < FR_STEPS; ++s) wf[j][s] = *reinterpret_cast<const u32x4 *>(p.w + wr * FR_K + k0 + 32 * s);
   }
-  if (!SWI) {
-#pragma unroll
-    for (int t = 0; t < XB; ++t)
-      old[t] = static_cast<const bf16_t *>(p.y)[static_cast<int64_t>(min(er + 16 * t, M - 1)) * p.N + n0 + ec];
-  }
+  if (!SWI) old = *dst;
   asm volatile("" ::: "memory");  // every load is issued by here (the compiler would sink them to their uses)
-  if (SWI) {  // the rounding points of pg_normalise_rows
 #pragma unroll
-    for (int t = 0; t < XB; ++t) {
+  for (int t = 0; t < XB; ++t) {
+    if (SWI) {  // the rounding points of pg_normalise_rows
       float s4[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) s4[q] = (sq[t][q][0] + sq[t][q][1]) + (sq[t][q][2] + sq[t][q][3]);
@@ -1400,52 +1402,46 @@ __global__ __launch_bounds__(64 * FR_WAVES) void few_rows_kernel(const SkinnyArg
         for (int e = 0; e < 4; ++e)
           xf[t][s][e] = pack_bf(lo_bf(xf[t][s][e]) * rn * lo_bf(nw[s][e]), hi_bf(xf[t][s][e]) * rn * hi_bf(nw[s][e]));
     }
+#pragma unroll
+    for (int s = 0; s < FR_STEPS; ++s) frag[2 + t][FR_STEPS * wid + s][lane] = xf[t][s];
   }
 #pragma unroll
-  for (int t = 0; t < XB; ++t)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < FR_STEPS; ++s)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[j][s]),
-                                                      __builtin_bit_cast(bf16x8, xf[t][s]), acc, 0, 0, 0);
-      // lane: x row 16 t + fr, weight rows 4 fg .. + 3 of block j
-      *reinterpret_cast<f32x4 *>(&part[((wid * XB + t) * 16 + fr) * PITCH + 16 * j + 4 * fg]) = acc;
-    }
+    for (int s = 0; s < FR_STEPS; ++s) frag[j][FR_STEPS * wid + s][lane] = wf[j][s];
   __syncthreads();
-  auto total = [&](int t, int col) {
-    float v = 0.f;
+  if (wid < 2 * XB * PARTS) {  // a chain: weight block j, x block t, part h of K
+    constexpr int N = FR_KSTEPS / PARTS;
+    const int j = wid & 1, t = XB == 1 ? 0 : wid >> 1, h = XB == 1 ? wid >> 1 : 0;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < FR_WAVES; ++w) v += part[((w * XB + t) * 16 + er) * PITCH + col];
-    return v;
-  };
+    for (int s = 0; s < N; ++s)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, frag[j][N * h + s][lane]),
+                                                    __builtin_bit_cast(bf16x8, frag[2 + t][N * h + s][lane]), acc, 0, 0, 0);
+    // lane: x row 16 t + fr, weight rows 4 fg .. + 3 of block j
+    *reinterpret_cast<f32x4 *>(&part[h][(16 * t + fr) * PITCH + 16 * j + 4 * fg]) = acc;
+  }
+  __syncthreads();
+  const bool live = row < M;
+  if (SWI) {
+    if (row >= 16 * XB || !live) return;  // (XB = 1: threads 0 .. 255 have an output)
+    const float g = round_bf(part[0][row * PITCH + col]), u = round_bf(part[0][row * PITCH + 16 + col]);
+    *dst = f2bf(round_bf(g / (1.0f + __expf(-g))) * u);
+  } else {
+    const bf16_t o = f2bf(bf2f(old) + round_bf(part[0][row * PITCH + col] + part[PARTS - 1][row * PITCH + col]));
+    if (live) *dst = o;
+    if (p.ss_out) {  // neighbouring columns first, as the epilogues whose lanes hold four of them
+      float ss = bf2f(o) * bf2f(o);
 #pragma unroll
-  for (int t = 0; t < XB; ++t) {
-    const int64_t row = er + 16 * t;
-    const bool live = row < M;
-    bf16_t *dst = static_cast<bf16_t *>(p.y) + row * p.N + n0 + ec;
-    if (SWI) {
-      if (tid < 256 && live) {
-        const float g = round_bf(total(t, ec)), u = round_bf(total(t, 16 + ec));
-        *dst = f2bf(round_bf(g / (1.0f + __expf(-g))) * u);
-      }
-    } else {
-      const bf16_t o = f2bf(bf2f(old[t]) + round_bf(total(t, ec)));
-      if (live) *dst = o;
-      if (p.ss_out) {
-        const float f = bf2f(o), ss = group_sum<32>(f * f);
-        if (live && ec == 0) p.ss_out[row * PG_SS_N + blockIdx.x] = ss;
-      }
+      for (int d = 1; d < 32; d <<= 1) ss += __shfl_xor(ss, d, 64);
+      if (live && col == 0) p.ss_out[row * PG_SS_N + blockIdx.x] = ss;
     }
   }
 }
 
-template <int EPI>
-static int launch_few_rows(const SkinnyArgs &a, hipStream_t s) {
-  const unsigned n = static_cast<unsigned>(a.N / (EPI == EPI_SWIGLU ? 16 : 32));
-  auto kern = a.M <= 16 ? few_rows_kernel<EPI, 1> : few_rows_kernel<EPI, 2>;
-  kern<<<n, 64 * FR_WAVES, 0, s>>>(a);
+static int launch_few_rows_swiglu(const SkinnyArgs &a, hipStream_t s) {
+  auto kern = a.M <= 16 ? few_rows_kernel<EPI_SWIGLU, 1> : few_rows_kernel<EPI_SWIGLU, 2>;
+  kern<<<static_cast<unsigned>(a.N / 16), 64 * FR_WAVES, 0, s>>>(a);
   return VK_OK;
 }
 
@@ -1515,7 +1511,7 @@ extern "C" int vk_norm_linear(const void *x, const void *norm_w, float eps, cons
                  PG_NORM_K);
     // 32 x 96 SwiGLU tiles while they fit one resident round of the chip (the decode step's 512 rows)
     const bool wide = swiglu && N % GW_BN == 0 && ((M + GW_BM - 1) / GW_BM) * (N / GW_BN) <= device_cus_cached();
-    rc = swiglu && M <= FR_ROWS && N % 16 == 0 ? launch_few_rows<EPI_SWIGLU>(p, s)
+    rc = swiglu && M <= FR_ROWS && N % 16 == 0 ? launch_few_rows_swiglu(p, s)
          : wide ? launch_gate_up_wide(p, s)
          : swiglu ? launch_panel<PRO_NORM_SS, EPI_SWIGLU>(p, s)
                   : (out_dtype == VK_DTYPE_F32 ? launch_panel<PRO_NORM_SS, EPI_F32>(p, s)
@@ -1560,11 +1556,16 @@ extern "C" int vk_linear_residual(const void *a, const void *w, void *x, int64_t
                "linear_residual: row sums of squares need K %% 64 == 0 and N = %d", PG_NORM_K);
   // 32 x 32 tiles while they fit one resident round of the chip (the decode step's 512 rows), else the panel
   const int64_t rs_tiles = ((M + RS_BM - 1) / RS_BM) * ((N + RS_BN - 1) / RS_BN);
-  const int rc = M <= 16 && K == FR_K && N % 32 == 0 ? launch_few_rows<EPI_RESID>(p, VK_STREAM(stream))
-                 : (K % (2 * PG_BK) == 0 && rs_tiles <= device_cus_cached())
-                     ? launch_resid(p, VK_STREAM(stream))
-                     : (panel_ok(p, PRO_NONE) ? launch_panel<PRO_NONE, EPI_RESID>(p, VK_STREAM(stream))
-                                              : dispatch_k<32, PRO_NONE, EPI_RESID>(p, VK_STREAM(stream)));
+  hipStream_t s = VK_STREAM(stream);
+  int rc = VK_OK;
+  if (K % (2 * PG_BK) == 0 && rs_tiles <= device_cus_cached()) {
+    if (M <= FR_RES_ROWS && K == FR_K && N % 32 == 0)
+      few_rows_kernel<EPI_RESID, 1><<<static_cast<unsigned>(N / 32), 64 * FR_WAVES, 0, s>>>(p);
+    else
+      rc = launch_resid(p, s);
+  } else {
+    rc = panel_ok(p, PRO_NONE) ? launch_panel<PRO_NONE, EPI_RESID>(p, s) : dispatch_k<32, PRO_NONE, EPI_RESID>(p, s);
+  }
   if (rc != VK_OK) return rc;
   return launch_status("linear_residual");
 }
