@@ -1159,6 +1159,32 @@ def test_decode_attention_split_merge(B, S):
     assert (out.float().cpu() - _sdpa_ref(q, k, v, lens)).abs().max() < 1e-2
 
 
+@pytest.mark.parametrize("B,S", [(128, 700), (4, 2081), (2, 70 * 256 + 31)])
+def test_decode_attention_merge_order(B, S):
+    """The merge adds the key splits' sums and outputs in their order (fused multiply-adds, weights from the maximum over
+    all splits), whatever their number: recomputed from the partials the workspace holds, bit for bit. (Another order
+    shows in about one output in 200000: 16 queries per sequence.)"""
+    g = torch.Generator(device=DEV).manual_seed(S + B)
+    k, v = (torch.randn(B, S, 2, 64, generator=g, device=DEV).to(BF) for _ in range(2))
+    lens = torch.randint(S // 2, S + 1, (B,), generator=g, device=DEV).int()
+    ws = ops.decode_attention_workspace(B, 8, S, DEV).view(torch.float32)
+    splits = ws.numel() // (B * 8 * 66)
+    ml = ws[B * splits * 512:].view(B, splits, 8, 2)
+    o = ws[:B * splits * 512].view(B, splits, 8, 64)
+    assert splits > 2
+    for _ in range(16):
+        q = torch.randn(B, 8, 64, generator=g, device=DEV).to(BF)
+        ws.zero_()
+        ml[..., 0] = float("-inf")  # (splits past a sequence's length: weight 0)
+        out = ops.decode_attention(q, k, v, lens, workspace=ws)
+        w = torch.exp2(ml[..., 0] - ml[..., 0].amax(1, keepdim=True)).double()
+        L, N = torch.zeros(B, 8, device=DEV), torch.zeros(B, 8, 64, device=DEV)
+        for s in range(splits):  # a product of two fp32 values is exact in fp64
+            L = (w[:, s] * ml[:, s, :, 1] + L.double()).float()
+            N = (w[:, s, :, None] * o[:, s] + N.double()).float()
+        assert torch.equal(out, (N / L[..., None]).to(BF))
+
+
 def test_select_update_with_final_norm():
     g = gen(99)
     B, d, V = 64, 512, 7

@@ -269,32 +269,45 @@ __global__ __launch_bounds__(DA_H * DA_D) void decode_attn_combine(const float *
   const int ntiles = static_cast<int>((len + DA_TILE - 1) / DA_TILE);
   const int nvalid = min(nsplit, (ntiles + tps - 1) / tps);
   // a wavefront per head: lane s holds split s's (max, sum), 64 splits at a time, and eight splits' outputs are in
-  // flight at once (one split after another, each behind two round trips: 5.5 -> 4.6 us for 9 splits)
+  // flight at once (one split after another, each behind two round trips: 5.5 -> 4.6 us for 9 splits). The sums run over
+  // the splits in order, with the weights taken from the maximum over all of them.
   const int lane = threadIdx.x & 63;
-  float M = -INFINITY, L = 0.f, N = 0.f;
-  for (int s0 = 0; s0 < nvalid; s0 += 64) {
-    const int n = min(64, nvalid - s0);
-    const int64_t base = (b * nsplit + s0) * DA_H + h;
-    const int64_t mine = base + static_cast<int64_t>(min(lane, n - 1)) * DA_H;
-    const float m_l = ws_ml[mine * 2], l_l = ws_ml[mine * 2 + 1];
-    constexpr int U = 8;
-    float o[U];
+  const int64_t base = b * nsplit * DA_H + h;
+  constexpr int U = 8;
+  auto ml_at = [&](int s0, float &m, float &l) {
+    const int64_t at = (base + static_cast<int64_t>(min(s0 + lane, nvalid - 1)) * DA_H) * 2;
+    m = ws_ml[at];
+    l = ws_ml[at + 1];
+  };
+  auto o_at = [&](int s) { return ws_o[(base + static_cast<int64_t>(min(s, nvalid - 1)) * DA_H) * DA_D + d]; };
+  float m, l, o[U];
+  ml_at(0, m, l);
 #pragma unroll
-    for (int u = 0; u < U; ++u) o[u] = ws_o[(base + static_cast<int64_t>(min(u, n - 1)) * DA_H) * DA_D + d];
-    const float m_new = fmaxf(M, wave_max(m_l));
-    const float keep = exp2f(M - m_new);
-    const float e_l = lane < n ? exp2f(m_l - m_new) : 0.f;
-    L = L * keep + wave_sum(e_l * l_l);
-    N *= keep;
-    M = m_new;
-    for (int s = 0; s < n; s += U) {
-      float nx[U];
+  for (int u = 0; u < U; ++u) o[u] = o_at(u);
+  float M = wave_max(m);
+  for (int s0 = 64; s0 < nvalid; s0 += 64) {
+    float mx, unused;
+    ml_at(s0, mx, unused);
+    M = fmaxf(M, wave_max(mx));
+  }
+  float e = exp2f(m - M), L = 0.f, N = 0.f;
+  for (int s = 0; s < nvalid; s += U) {
+    if (s > 0 && s % 64 == 0) {
+      ml_at(s, m, l);
+      e = exp2f(m - M);
+    }
+    float nx[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) nx[u] = ws_o[(base + static_cast<int64_t>(min(s + U + u, n - 1)) * DA_H) * DA_D + d];
+    for (int u = 0; u < U; ++u) nx[u] = o_at(s + U + u);
 #pragma unroll
-      for (int u = 0; u < U; ++u) N += __shfl(e_l, min(s + u, 63), 64) * (s + u < n ? o[u] : 0.f);
-#pragma unroll
-      for (int u = 0; u < U; ++u) o[u] = nx[u];
+    for (int u = 0; u < U; ++u) {
+      if (s + u < nvalid) {  // uniform
+        const int at = (s + u) % 64;
+        const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), at));
+        L += w * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l), at));
+        N += w * o[u];
+      }
+      o[u] = nx[u];
     }
   }
   out[(b * DA_H + h) * DA_D + d] = f2bf(N / L);
