@@ -254,3 +254,50 @@ def test_attention_and_prefill_plans_match_loop_forms():
         pp = PrefillPlan(seq, "cpu", keep=keep)
         cu = pp.cu
         assert pp.last_idx.tolist() == [cu[j + 1] - kk + i for j, kk in enumerate(keep) for i in range(kk)]
+
+
+_SLAB_CHECK = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "slab_loads.h"
+using namespace vk;
+int main() {
+  long bad = 0, n = 0;
+  // row blocks and wavefronts of the tile shapes (x and w; a SwiGLU half), every count of valid rows
+  const int shapes[][2] = {{256, 8}, {128, 4}, {128, 8}, {64, 4}, {64, 2}, {32, 2}};
+  for (auto &s : shapes)
+    for (uint32_t K : {64u, 192u, 512u, 3072u, 1u << 22})
+      for (int rows = 1; rows <= s[0]; ++rows) {
+        const uint64_t end = slab_bytes(rows, K);
+        const int nk = K / 64, slabs[] = {0, nk / 2, nk - 1};
+        for (int kt : slabs)
+          for (int wid = 0; wid < s[1]; ++wid)
+            for (int i = 0; i < s[0] / SLAB_ROWS / s[1]; ++i)
+              for (int lane = 0; lane < 64; ++lane) {
+                const int row = SLAB_ROWS * (wid + s[1] * i) + lane / 8;
+                const uint32_t vo = slab_vector_offset(wid, s[1], i, lane, K), so = slab_scalar_offset(kt);
+                const bool past = row >= rows;
+                const bool excluded = vo >= end;                            // the check leaves the scalar offset out
+                const bool wraps = vo >= static_cast<uint32_t>(end - so);   // 32-bit end minus scalar
+                const bool below = so > end;                                // (end minus scalar would wrap)
+                const uint64_t at = uint64_t(row) * K * 2 + uint64_t(kt) * 128, want = at + 128;
+                const bool inside = uint64_t(vo) + so >= at && uint64_t(vo) + so + 16 <= want && want <= end;
+                if (excluded != past || wraps != past || below || (!past && !inside)) ++bad;
+                ++n;
+              }
+      }
+  std::printf("%ld of %ld\n", bad, n);
+  return bad != 0;
+}
+"""
+
+
+def test_slab_loads_stay_inside_their_descriptor(tmp_path):
+    """The large products' direct loads: whether a buffer load's range check counts the scalar offset or not, a row inside
+    the descriptor is read at its own bytes and every row past its end is out of range."""
+    src, exe = tmp_path / "slab.cpp", tmp_path / "slab"
+    src.write_text(_SLAB_CHECK)
+    csrc = os.path.join(os.path.dirname(hip_ops.__file__), "csrc")
+    subprocess.run(["g++", "-O2", "-std=c++17", f"-I{csrc}", str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout

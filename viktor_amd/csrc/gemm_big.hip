@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "slab_loads.h"
 
 namespace vk {
 
@@ -57,7 +58,8 @@ using GbSquare = GbShape<2, 2, 4>;  // 128 x 128, 64 KB: two workgroups per CU
 typedef __attribute__((address_space(3))) void lds_void;
 
 // A buffer descriptor over `bytes` bytes from p (raw, unstrided), and one 16-byte direct buffer->LDS load per lane:
-// lane l reads p + vo + so (zero past the end) into dst + 16 l. Plain device functions: written in a kernel template
+// lane l reads p + vo + so into dst + 16 l (zero if that is past the end; slab_loads.h: for either reading of the range
+// check). Plain device functions: written in a kernel template
 // with arguments that depend on its parameters, the builtin makes the host pass drop the kernel's launch stub.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t gb_rsrc(const bf16_t *p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(p), 0, bytes, 0x00020000);
@@ -175,30 +177,29 @@ __global__ __launch_bounds__(64 * SH::WAVES, SH::WAVES_PER_SIMD) void gemm_big_k
   // cache line; with 64-byte rows the same stream ran at 16 instead of 24 TB/s). The stage holds a slab's
   // two 32-wide slices; a wavefront reads the next slice's fragments while this one's MFMAs run, from two
   // register sets. Once every wavefront has its fragments of slab kt in registers (the barrier), slab kt + 2
-  // goes into its stage; slab kt + 1 had the time of a whole slab to land. Buffer loads: rows past M or N are
-  // past the descriptor's end and read as zero (they only reach outputs that are not stored), and the K offset
-  // and row block ride in the scalar offset, so a source takes one register.
+  // goes into its stage; slab kt + 1 had the time of a whole slab to land. Buffer loads (offsets: slab_loads.h): rows
+  // past M or N are past the descriptor's end and read as zero (they only reach outputs that are not stored), and the K
+  // offset rides in the scalar offset, so a source takes one 32-bit register.
   // LDS slot of K chunk c (16 bytes) in row r: c ^ ((r >> 1) & 7), so 16 consecutive rows of a chunk cover all
   // 64 banks.
   const int64_t xrows = M - m0 < GB_BM ? M - m0 : GB_BM;
-  const auto xr = gb_rsrc(x + m0 * K, static_cast<uint32_t>(xrows) * K * 2);
+  const auto xr = gb_rsrc(x + m0 * K, slab_bytes(static_cast<uint32_t>(xrows), K));
   constexpr int HALVES = SWIGLU ? 2 : 1;  // SwiGLU: gate rows n0.. of w, then the matching up rows N + n0..
   const uint32_t wrows = N - n0 < SH::BW / HALVES ? N - n0 : SH::BW / HALVES;
-  const auto wr = gb_rsrc(w + static_cast<int64_t>(n0) * K, wrows * K * 2);
-  const auto wr2 = gb_rsrc(w + static_cast<int64_t>(SWIGLU ? N + n0 : n0) * K, wrows * K * 2);
-  const int lr = SH::RPL * wid + (lane >> 3);
-  const uint32_t vo = static_cast<uint32_t>(lr) * K * 2 + 16 * ((lane & 7) ^ ((lr >> 1) & 7));
-  const uint32_t rstep = SH::RPL * NWAVES * static_cast<uint32_t>(K) * 2;
+  const auto wr = gb_rsrc(w + static_cast<int64_t>(n0) * K, slab_bytes(wrows, K));
+  const auto wr2 = gb_rsrc(w + static_cast<int64_t>(SWIGLU ? N + n0 : n0) * K, slab_bytes(wrows, K));
+  static_assert(SH::RPL == SLAB_ROWS && GB_ROWB == SLAB_BYTES, "a direct load covers 8 rows of a slab");
   auto issue = [&](int stage, int kt) {
     char *base = smem + stage * GB_STAGEB;
-    const uint32_t so = static_cast<uint32_t>(kt) * 128;
+    const uint32_t so = slab_scalar_offset(kt);
 #pragma unroll
-    for (int i = 0; i < SH::XLOADS; ++i) gb_buf_lds(xr, base + (wid + NWAVES * i) * 1024, vo, so + i * rstep);
+    for (int i = 0; i < SH::XLOADS; ++i)
+      gb_buf_lds(xr, base + (wid + NWAVES * i) * 1024, slab_vector_offset(wid, NWAVES, i, lane, K), so);
 #pragma unroll
     for (int i = 0; i < SH::WLOADS; ++i) {
       constexpr int HL = SH::WLOADS / HALVES;
-      const int ih = i >= HL ? i - HL : i;
-      gb_buf_lds(i >= HL ? wr2 : wr, base + GB_XTILEB + (wid + NWAVES * i) * 1024, vo, so + ih * rstep);
+      gb_buf_lds(i >= HL ? wr2 : wr, base + GB_XTILEB + (wid + NWAVES * i) * 1024,
+                 slab_vector_offset(wid, NWAVES, i >= HL ? i - HL : i, lane, K), so);
     }
   };
   const int sw = 16 * (fg ^ ((fr >> 1) & 7));
