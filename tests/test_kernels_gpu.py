@@ -1011,6 +1011,35 @@ def test_linear_qkv_rope_fp32_norm_weights(M):
         assert (d > 0).float().mean() < 1e-3 and bf_close(a, b.float().cpu(), ulps=2, atol=2e-2)[0]
 
 
+@pytest.mark.parametrize("weights", ["none", "bf16", "f32"])
+def test_linear_qkv_rope_rounds_the_rotation_once_fused(weights):
+    """The rotation of the fp32-table Wqkv epilogues has one rounding, whatever the tile: y1 cos is fused into
+    y1 cos - rn(y2 sin), y2 cos into rn(y1 sin) + y2 cos. The unrotated rows are the same call's at table row 0 (cos 1,
+    sin 0); products of bf16 and fp32 values and their sums are formed in 64 bits and rounded to fp32, then to bf16."""
+    M, H, HKV, D, K = 4500, 8, 2, 64, 512
+    g = gen(61)
+    x = to_dev(R.bf(torch.randn(M, K, generator=g) * 2), BF)
+    wq = to_dev(R.bf(torch.randn((H + 2 * HKV) * D, K, generator=g) / math.sqrt(K)), BF)
+    nw = None if weights == "none" else to_dev(1 + 0.1 * torch.randn(D, generator=g), BF if weights == "bf16" else None)
+    cos, sin = (to_dev(t) for t in R.rope_tables(D, 4096, 1e6))
+    assert bool((cos[0] == 1).all()) and bool((sin[0] == 0).all())
+    rpos = to_dev(torch.randint(1, 4096, (M,), generator=g).int())
+
+    def rotated(pos):
+        q, k, _ = ops.linear_qkv_rope(x, wq, nw, nw, cos, sin, pos, None, None, None, 1e-6, H, HKV, D, return_kv=True)
+        return torch.cat([q, k], 1).float()
+
+    y, got = rotated(torch.zeros_like(rpos)).double(), rotated(rpos)
+    y1, y2 = y[..., :D // 2], y[..., D // 2:]
+    c, s = cos[rpos.long()].double()[:, None], sin[rpos.long()].double()[:, None]
+    rn = lambda t: t.float().double()
+    fused = torch.cat([y1 * c - rn(y2 * s), rn(y1 * s) + y2 * c], -1).float().to(BF).float()
+    other = torch.cat([rn(y1 * c) - y2 * s, y1 * s + rn(y2 * c)], -1).float().to(BF).float()
+    assert torch.equal(got, fused)
+    assert not torch.equal(got[..., :D // 2], other[..., :D // 2])  # (the inputs tell the two roundings apart)
+    assert not torch.equal(got[..., D // 2:], other[..., D // 2:])
+
+
 def test_linear_qkv_rope_no_norm_in_place():
     """The encoder's use: no QK-norm, rotary positions per row, q / k / v written back into the packed qkv rows."""
     g = gen(11)

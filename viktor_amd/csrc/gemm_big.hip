@@ -515,9 +515,11 @@ __global__ __launch_bounds__(64 * SH::WAVES, SH::WAVES_PER_SIMD) void gemm_big_k
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+              // (which product is fused into the sum is written out: with fp32 tables both are inexact, and the compiler
+              // chose another one in each tile shape)
               const float y1 = v[i][e], y2 = v[i + 2][e];
-              v[i][e] = y1 * cs[e] - y2 * sn[e];
-              v[i + 2][e] = y1 * sn[e] + y2 * cs[e];
+              v[i][e] = __builtin_fmaf(y1, cs[e], -(y2 * sn[e]));
+              v[i + 2][e] = __builtin_fmaf(y2, cs[e], y1 * sn[e]);
             }
           }
         }
@@ -646,8 +648,8 @@ static int launch_big(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int 
   // 128, 64 x 64 tiles: M = 1324 (44 tiles of 128 x 128) 9.3 / 15.7 / 22.6, 8.1 / 10.5 / 18.6, 8.3 / 9.3 / 10.9; 4099
   // (132) 9.7 / 21.1 / 24.3, 8.5 / 17.0 / 21.4, 8.6 / 17.4 / 21.7; 7500 (236) 10.0 / 21.4 / 25.6, 9.3 / 18.8 / 22.8,
   // 10.6 / 21.1 / 25.6; 9000 (284) 13.7 / 25.4 / 29.4, 11.9 / 26.6 / 30.6, 13.5 / 31.3 / 38.8. The Wqkv epilogues keep
-  // one shape: the compiler contracts their fp32 rotation differently in another, and a row's bits are not to depend on
-  // the batch.
+  // the one shape: 64 x 128 tiles at M = 4099 take 12.5 us with bf16 tables and a cache, 10.5 with fp32 ones, 11.0 with
+  // fp32 weights and the kept product, 15.9 at N = 1536 without norm, against 12.4, 10.5, 12.3 and 13.9.
   if constexpr (EPI != GB_QKV && EPI != GB_QKV_BF16 && EPI != GB_QKV_W32) {
     constexpr int OUT_COLS = EPI == GB_SWIGLU ? GbSquare::BW / 2 : GbSquare::BW;
     const int64_t tiles = (M + GbSquare::BM - 1) / GbSquare::BM * ((N + OUT_COLS - 1) / OUT_COLS);
