@@ -12,7 +12,7 @@
 //   * Against 256 x 128 tiles with 32-wide slabs in a three-stage ring (same box, us): N = 512, K = 512 / 1536 + bf16
 //     residual at M = 4099: 18.5 / 35.1 -> 11.2 / 20.4, M = 45057: 46.0 / 92.5 -> 40.7 / 77.7, M = 131136: 122 / 278
 //     -> 111 / 269; SwiGLU N = 1536, K = 512: 20.5 -> 17.8, 154 -> 146, 427 -> 417; Wqkv N = 768: M = 45057 62 -> 53,
-//     M = 131136 153 -> 160 (the one shape that lost).
+//     M = 131136 see launch_big_shape.
 //   * Tiles are ordered XCD-aware: workgroup p runs on XCD p % 8, so each XCD gets a contiguous range of
 //     tiles and the N-tiles that share a block of x rows share that XCD's L2.
 //   * The product is formed transposed, C^T = W X^T (the weight fragment is the MFMA A operand), so each
@@ -625,7 +625,16 @@ static int launch_big_shape(const bf16_t *x, const bf16_t *w, void *y, int64_t M
   // Row blocks per group of the tile order: an XCD has 64 workgroups resident, 16 x 4 tiles for few column blocks
   // (M = 131136, N = 512, K = 1536: 230 -> 198 us for the loop alone against groups of 8); while an XCD's share is
   // below a few such groups, 8 (M = 9000, N = 512, K = 3072: 48 -> 41 us against 16).
-  const int group_m = tiles_n <= 4 && total >= 2048 ? 16 : 8;
+  // The Wqkv products (6 column blocks and more) take 16 as well once their rows in and out outgrow the 256 MB last-level
+  // cache: M = 131136 with groups of 8 and 16 (in brackets: 256 x 128 tiles in groups of 8, the same rows as 16 here) N =
+  // 1536 310 and 301 us (305), fp32 weights and the kept product 220 and 214 (214), fp32 tables 166 and 164 (161), bf16
+  // tables and a cache 177 and 176 (172), at M = 90000 112 and 108 (109). Below it 8: M = 45057 97 and 98, 70 and 72, 57
+  // and 59, 56 and 59.
+  int64_t row_cols = 0;
+  if constexpr (EPI == GB_QKV || EPI == GB_QKV_BF16 || EPI == GB_QKV_W32)
+    row_cols = K + 64 * qa.H + 128 * qa.HKV * ((qa.ko != nullptr) + (qa.kc != nullptr)) + (qa.raw != nullptr ? N : 0);
+  const bool big_rows = M * row_cols * 2 > (int64_t(256) << 20);
+  const int group_m = big_rows || (tiles_n <= 4 && total >= 2048) ? 16 : 8;
   gemm_big_kernel<EPI, SH><<<static_cast<unsigned>(total), 64 * SH::WAVES, SH::SMEM, s>>>(
       x, w, y, M, N, K, tiles_n, static_cast<int>(total), group_m, qa);
   return VK_OK;
