@@ -90,6 +90,7 @@ def gspo_rewards(calls: List[str], labels: List[str], weights: List[np.ndarray],
 def _bases(tokens: torch.Tensor, tokenizer):
     """The base strings of output tokens [N, T] on the device (vk_tokens_to_bases): rows [N, T k] uint8 and their
     lengths [N] int32. No host synchronisation."""
+    require_device(tokens, "output tokens to bases")
     N, T = tokens.shape
     V, k = tokenizer.vocab_size, tokenizer.k
     strings = [b"" if t < N_SPECIAL else tokenizer.strings[t].encode() for t in range(V)]
@@ -105,7 +106,10 @@ def _bases(tokens: torch.Tensor, tokenizer):
 def calls_from_tokens(tokens: torch.Tensor, tokenizer):
     """Device base strings of the engine's output tokens [N, T] (int64): the tokenizer's decode on the device
     (stops at the first EOS, skips PAD and BOS; a token writes its k-mer or tail). Returns (bytes [total] uint8,
-    offsets [N] int64, lengths [N] int32, max length)."""
+    offsets [N] int64, lengths [N] int32, max length). Host tokens are decoded on the host."""
+    if not tokens.is_cuda:
+        ids = tokens.clamp(0, tokenizer.vocab_size - 1).tolist()
+        return _pack([tokenizer.decode(r).encode() for r in ids], tokens.device)
     rows, lens = _bases(tokens, tokenizer)
     offsets = torch.cumsum(lens.long(), 0) - lens
     out = rows[torch.arange(rows.shape[1], device=rows.device) < lens[:, None]]
@@ -118,7 +122,6 @@ def gspo_rewards_from_tokens(tokens: torch.Tensor, tokenizer, labels: List[str],
                              empty_max=EMPTY_MAX):
     """The rollout's rewards straight from the engine's device output (no host decode): tokens [windows * G, T];
     returns the device dict of strict_identity (reward [windows * G] fp32)."""
-    require_device(tokens, "gspo_rewards_from_tokens")
     rows, lens = _bases(tokens, tokenizer)
     N, width = rows.shape
     # rows longer than the kernel's longest call: only then the lengths are read back
