@@ -386,7 +386,8 @@ int vk_attention_backward_prefixed(const void *q, const void *k, const void *v, 
  * sequence's query rows from its row `first row` (>= the first key); slot < 0 writes dk / dv (a block that is one
  * entry), slot >= 0 the partial block `slot` of part_k / part_v ([slots, 128, HKV, D] fp32, a caller's workspace, no
  * initial value). red holds n_red entries (first packed row, keys, first slot, slots): the split blocks, whose partial
- * blocks are summed in slot order into dk / dv. No reference counterpart of its own (the same sums, regrouped).
+ * blocks are summed in slot order into dk / dv; red, part_k and part_v may not be NULL. No reference counterpart of its
+ * own (the same sums, regrouped).
  */
 int vk_attention_backward_chunked(const void *q, const void *k, const void *v, const void *out, const void *dout,
                                   const float *lse, const int32_t *cu, int32_t n_seq, const int32_t *q_plan,

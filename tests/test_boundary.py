@@ -81,6 +81,11 @@ def test_argument_errors_return_status_without_device_work():
     assert rc == 1 and b"fp32 rotary tables" in lib.vk_last_error()
     rc = lib.vk_rmsnorm_backward(p, 1, p, 0, p, 0, None, p, None, p, 4, 512, 1e-6, None)  # fp32 x with bf16 weights
     assert rc == 3
+    # chunked key blocks without partial buffers, also with an empty list of sums (the plan's slots are read on the device)
+    a = ctypes.c_void_p(p.value + -p.value % 16)
+    rc = lib.vk_attention_backward_chunked(a, a, a, a, a, a, a, 1, a, 0, a, 1, 0, 128, a, 0, None, None, a, a, a, a, 8, 2,
+                                           64, None)
+    assert rc == 1 and b"partial buffers" in lib.vk_last_error()
     rc = lib.vk_timestamp(None, 0, None)
     assert rc == 1 and b"null" in lib.vk_last_error()
     rc = lib.vk_timestamp(p, -1, None)

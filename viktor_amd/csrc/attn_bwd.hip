@@ -601,7 +601,8 @@ extern "C" int vk_attention_backward_chunked(const void *q, const void *k, const
                                              int32_t n_kblocks, int64_t n_rows, int64_t stride_tok, const int32_t *red,
                                              int32_t n_red, float *part_k, float *part_v, float *dd, float *dq,
                                              float *dk, float *dv, int32_t H, int32_t HKV, int32_t D, void *stream) {
-  VK_CHECK_ARG(n_red >= 0 && (n_red == 0 || (red && part_k && part_v && vk_aligned16(part_k) && vk_aligned16(part_v))),
+  // (whatever n_red is: a plan entry's slot says where a block goes, and it is read on the device)
+  VK_CHECK_ARG(n_red >= 0 && red && part_k && part_v && vk_aligned16(part_k) && vk_aligned16(part_v),
                "attention_backward_chunked: partial buffers");
   const AbPrefix pre{nullptr, nullptr, part_k, part_v, 0};
   const AbChunks chunks{red, n_red};
