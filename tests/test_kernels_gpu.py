@@ -198,25 +198,27 @@ def test_small_batch_tiles_same_bits(M):
 
 def test_linear_wide_tiles_same_bits():
     """256 row blocks of 256 fill the chip with 256 x 256 tiles at K >= 1024; a row's bits are those of the 128 x 128
-    tiles that a smaller batch runs."""
+    tiles that 16500 rows run (258 of them, while 65 wide ones would leave most CUs idle) and of the 64 x 64 tiles of
+    4133 rows."""
     g = gen(77)
-    M, N, K = 65536 - 37, 248, 1088
-    x = to_dev(R.bf(torch.randn(4133, K, generator=g)), BF)
+    M, mid, few, N, K = 65536 - 37, 16500, 4133, 248, 1088
+    x = to_dev(R.bf(torch.randn(mid, K, generator=g)), BF)
     w = to_dev(R.bf(torch.randn(N, K, generator=g) / math.sqrt(K)), BF)
-    rows = torch.arange(M, device=DEV) % 4133
+    rows = torch.arange(M, device=DEV) % mid
     big = x[rows]
-    small = ops.linear(x, w)
-    assert torch.equal(ops.linear(big, w), small[rows])
-    small = ops.linear(x, w, out_dtype=torch.float32)
-    assert torch.equal(ops.linear(big, w, out_dtype=torch.float32), small[rows])
-    assert torch.allclose(small.double(), x.double() @ w.double().t(), rtol=1e-5, atol=1e-5)
+    for dt in (BF, torch.float32):
+        square = ops.linear(x, w, out_dtype=dt)
+        assert torch.equal(ops.linear(big, w, out_dtype=dt), square[rows])
+        assert torch.equal(ops.linear(x[:few], w, out_dtype=dt), square[:few])
+    assert torch.allclose(square.double(), x.double() @ w.double().t(), rtol=1e-5, atol=1e-5)
 
 
 @pytest.mark.parametrize("M,N,K", [(4099, 1536, 512), (8192, 520, 512), (4608, 512, 1536), (5000, 3072, 1024)])
 def test_linear_large_m_tile_shapes_same_bits(M, N, K):
-    """Large M: bf16 outputs run 256 x 256 tiles, fp32 outputs at K < 1024 the 256 x 128 tiles; both accumulate
-    every output in the same K order, so the bf16 result is the fp32 result rounded, bit for bit (partial row
-    and column tiles included)."""
+    """Large M, partial row and column tiles included: the bf16 result is the fp32 result rounded, bit for bit, and the
+    first rows alone, in fewer and mostly smaller tiles (128 x 128 whole against 64 x 64 and 64 x 128; 64 x 128 against
+    64 x 64; 256 x 256 against 128 x 128 and 64 x 128), have the same bits."""
+    from viktor_amd._lib import call, ptr, stream_handle
     g = gen(M + 3 * N + K)
     x = to_dev(R.bf(torch.randn(M, K, generator=g)), BF)
     w = to_dev(R.bf(torch.randn(N, K, generator=g) / math.sqrt(K)), BF)
@@ -225,6 +227,10 @@ def test_linear_large_m_tile_shapes_same_bits(M, N, K):
     assert torch.equal(y, y32.to(BF))
     ref = x.double() @ w.double().t()
     assert torch.allclose(y32.double(), ref, rtol=1e-5, atol=1e-5)
+    for m in (1000, 2000, 4097):
+        part = torch.empty(m, N, dtype=torch.float32, device=DEV)
+        call("vk_gemm_rows", ptr(x), ptr(w), ptr(part), m, N, K, 1, stream_handle())
+        assert torch.equal(part, y32[:m])
 
 
 @pytest.mark.parametrize("M", [1, 100, 512, 4500])

@@ -9,6 +9,7 @@ import torch
 
 from oracle import reference as R
 from viktor_amd import reward as RW
+from viktor_amd._lib import HipLibraryError
 from viktor_amd.tokenizer import KmerTokenizer
 
 pytestmark = pytest.mark.gpu
@@ -123,7 +124,7 @@ def test_strict_identity_at_the_edges_of_column_blocks(m):
     scored = [rng.random(len(l)) > 0.3 for l in labels]
     calls = ["".join(rng.choice(list("ACGT"), n)) for n in (127, 128, 191, 192, 193, 447, 448, 449)]
     calls += [_mutate(rng, labels[0], 0.1), _mutate(rng, labels[1], 0.4)]
-    if m in (512, 4095):
+    if m in (257, 2049):
         calls.append("".join(rng.choice(list("ACGT"), 8192)))
     _check(calls, labels, scored, [i % 2 for i in range(len(calls))])
 
@@ -145,3 +146,23 @@ def test_token_rows_at_the_edges_of_a_pass(k, T):
     want = [tok.decode(r.tolist()) for r in rows.clamp(0, tok.vocab_size - 1)]
     assert [bytes(got[o:o + n]).decode() for o, n in zip(off, lens)] == want
     assert longest == max(len(w) for w in want)
+
+
+def test_rewards_from_token_rows_wider_than_a_call():
+    """Rows of more than 8192 bytes, which is the longest call: the lengths are read back, short calls in such rows score
+    as their strings do, and a call that is longer is refused."""
+    rng = np.random.default_rng(6)
+    tok = KmerTokenizer(4)
+    G, T = 2, 2050
+    labels = ["".join(rng.choice(list("ACGT"), n)) for n in (300, 41)]
+    weights = [rng.random(len(l)) for l in labels]
+    rows = torch.tensor(rng.integers(3, tok.vocab_size, (2 * G, T)), dtype=torch.long)
+    for b, n in enumerate((70, 0, 12, 2047)):
+        rows[b, n] = 2
+    assert T * tok.k > RW.MAX_CALL
+    got = RW.gspo_rewards_from_tokens(rows.to(DEV), tok, labels, weights, G)["reward"]
+    host = RW.gspo_rewards([tok.decode(r.tolist()) for r in rows], labels, weights, G, device=DEV)
+    assert np.array_equal(got.double().cpu().numpy().reshape(-1, G), host)
+    rows[:, :] = 3
+    with pytest.raises(HipLibraryError, match="8192"):
+        RW.gspo_rewards_from_tokens(rows.to(DEV), tok, labels, weights, G)
