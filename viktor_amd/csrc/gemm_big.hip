@@ -414,8 +414,7 @@ __global__ __launch_bounds__(64 * SH::WAVES, SH::WAVES_PER_SIMD) void gemm_big_k
       const int j = pass * (PASS_ROWS / 16) + jj;
       char *rowp = stg + (16 * jj + fr) * PITCH;
       if (RESID) {
-        // lane: row 16 j + fr, columns qcol0 + 16 i + 4 fg + e; the old residual is read right here (each element
-        // by the lane that overwrites it)
+        // lane: row 16 j + fr, columns qcol0 + 16 i + 4 fg + e (the same elements prefetch read for it)
         int64_t rrow = qrow0 + 16 * j + fr;
         const bool live = rrow < M;
         rrow = live ? rrow : M - 1;
@@ -656,7 +655,10 @@ static int launch_big(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int 
   // and more, shorter chains run side by side. Residual product N = 512, K = 512 / 1536 / 2048, us with 128 x 128, 64 x
   // 128, 64 x 64 tiles: M = 1324 (44 tiles of 128 x 128) 9.3 / 15.7 / 22.6, 8.1 / 10.5 / 18.6, 8.3 / 9.3 / 10.9; 4099
   // (132) 9.7 / 21.1 / 24.3, 8.5 / 17.0 / 21.4, 8.6 / 17.4 / 21.7; 7500 (236) 10.0 / 21.4 / 25.6, 9.3 / 18.8 / 22.8,
-  // 10.6 / 21.1 / 25.6; 9000 (284) 13.7 / 25.4 / 29.4, 11.9 / 26.6 / 30.6, 13.5 / 31.3 / 38.8. The Wqkv epilogues keep
+  // 10.6 / 21.1 / 25.6; 9000 (284) 13.7 / 25.4 / 29.4, 11.9 / 26.6 / 30.6, 13.5 / 31.3 / 38.8. The plain and fp32
+  // epilogues go the same way (N = 512, bf16 out, K = 512 / 1536 / 3072: M = 4099 6.2 / 17.3 / 32.4, 6.1 / 12.0 / 27.0, 6.1 /
+  // 14.7 / 26.7; 7500 6.5 / 18.6 / 33.3, 6.3 / 17.0 / 29.9, 7.1 / 18.9 / 33.9; fp32 out, K = 512: 6.9, 6.6, 6.4 and 7.5, 7.0,
+  // 7.6); the SwiGLU product of N = 1536 has more tiles than CUs from M = 1281 on. The Wqkv epilogues keep
   // the one shape: 64 x 128 tiles at M = 4099 take 12.5 us with bf16 tables and a cache, 10.5 with fp32 ones, 11.0 with
   // fp32 weights and the kept product, 15.9 at N = 1536 without norm, against 12.4, 10.5, 12.3 and 13.9.
   if constexpr (EPI != GB_QKV && EPI != GB_QKV_BF16 && EPI != GB_QKV_W32) {
@@ -669,8 +671,8 @@ static int launch_big(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int 
   return launch_big_shape<EPI, GbSquare>(x, w, y, M, N, K, qa, s);
 }
 
-// Entry used by vk_linear for large M and by vk_gemm_rows (K % 64 == 0: an even number of K slices; N % 8 == 0:
-// whole 16-byte output chunks).
+// Entry used by vk_linear for large M and by vk_gemm_rows (K % 64 == 0: whole slabs, of any count; N % 8 == 0: whole
+// 16-byte output chunks).
 int gemm_big(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int N, int K, bool swiglu, bool out_f32,
              hipStream_t s) {
   const GbQkv none{};

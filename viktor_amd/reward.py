@@ -3,7 +3,7 @@
 Reference: scripts/gspo.py:86-89 (strict_identity), 446 (the reward of a rollout), scripts/train.py:170-188
 (ref_errors, the edlib NW path's error positions), scripts/evaluate.py:30 (EMPTY_MAX). The reference runs
 edlib on the host, one call after another; here one kernel scores every call of a rollout at once
-(vk_strict_identity: the edit-distance DP as a systolic array, 512 label rows per wavefront).
+(vk_strict_identity: the edit-distance DP as a systolic array, 256 label rows per wavefront).
 
 The alignment path behind the error positions: at every cell the first optimal predecessor in the order
 diagonal, deletion, insertion. edlib's own traceback order is not available here; the edit distance, and
