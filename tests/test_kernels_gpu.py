@@ -1046,6 +1046,34 @@ def test_linear_qkv_rope_rounds_the_rotation_once_fused(weights):
     assert not torch.equal(got[..., D // 2:], other[..., D // 2:])
 
 
+@pytest.mark.parametrize("form", ["tables_bf16", "tables_f32", "weights_f32"])
+def test_linear_qkv_rope_wide_tiles_same_bits(form):
+    """Wqkv batches of 16385 to 21845 rows run 256 x 256 tiles: q, k, v, the cache rows and the kept product have the bits of
+    the same rows in a batch of 128 x 128 ones, the last row block is partial, and nothing is stored past the last row."""
+    M, few, H, HKV, D, K, S = 20003, 5001, 8, 2, 64, 512, 64
+    g = gen(83)
+    x = to_dev(R.bf(torch.randn(M, K, generator=g) * 2), BF)
+    wq = to_dev(R.bf(torch.randn((H + 2 * HKV) * D, K, generator=g) / math.sqrt(K)), BF)
+    nw = to_dev(1 + 0.1 * torch.randn(D, generator=g), None if form == "weights_f32" else BF)
+    cos, sin = (to_dev(t, BF if form == "tables_bf16" else None) for t in R.rope_tables(D, 4096, 1e6))
+    rpos = to_dev(torch.randint(0, 4096, (M,), generator=g).int())
+    row = torch.arange(M, device=DEV).int()
+
+    def run(n):
+        caches = [torch.full((M // S + 1, S, HKV, D), 7.0, dtype=BF, device=DEV) for _ in range(2)]
+        raw = torch.full((n + 1, (H + 2 * HKV) * D), 7.0, dtype=BF, device=DEV)
+        out = [torch.full((n + 1, h * D), 7.0, dtype=BF, device=DEV) for h in (H, HKV, HKV)]
+        ops.linear_qkv_rope(x[:n], wq, nw, nw, cos, sin, row[:n] % S, row[:n] // S, *caches, 1e-6, H, HKV, D,
+                            return_kv=True, rope_pos=rpos[:n], q_out=out[0][:n], kv_out=(out[1][:n], out[2][:n]),
+                            qkv_out=raw[:n])
+        return [*out, raw, *(c.view(-1, HKV * D)[:n + 1] for c in caches)]
+
+    for whole, part in zip(run(M), run(few)):
+        assert torch.equal(whole[:few], part[:few])
+        assert bool((whole[M] == 7.0).all()) and bool((part[few] == 7.0).all())
+    assert torch.equal(run(M)[3][:M], ops.linear(x, wq))
+
+
 def test_linear_qkv_rope_no_norm_in_place():
     """The encoder's use: no QK-norm, rotary positions per row, q / k / v written back into the packed qkv rows."""
     g = gen(11)

@@ -621,35 +621,65 @@ static int launch_big_shape(const bf16_t *x, const bf16_t *w, void *y, int64_t M
   if (total >= (int64_t(1) << 31)) return fail(VK_ERR_ARG, "linear: too many tiles");
   // (the descriptors hold a row block's bytes in 32 bits)
   if (K > (1 << 22)) return fail(VK_ERR_ARG, "linear: K %d too large", K);
-  // Row blocks per group of the tile order: an XCD has 64 workgroups resident, 16 x 4 tiles for few column blocks
-  // (M = 131136, N = 512, K = 1536: 230 -> 198 us for the loop alone against groups of 8); while an XCD's share is
-  // below a few such groups, 8 (M = 9000, N = 512, K = 3072: 48 -> 41 us against 16).
-  // The Wqkv products (6 column blocks and more) take 16 as well once their rows in and out outgrow the 256 MB last-level
-  // cache: M = 131136 with groups of 8 and 16 (in brackets: 256 x 128 tiles in groups of 8, the same rows as 16 here) N =
-  // 1536 310 and 301 us (305), fp32 weights and the kept product 220 and 214 (214), fp32 tables 166 and 164 (161), bf16
-  // tables and a cache 177 and 176 (172), at M = 90000 112 and 108 (109). Below it 8: M = 45057 97 and 98, 70 and 72, 57
-  // and 59, 56 and 59.
-  int64_t row_cols = 0;
-  if constexpr (EPI == GB_QKV || EPI == GB_QKV_BF16 || EPI == GB_QKV_W32)
-    row_cols = K + 64 * qa.H + 128 * qa.HKV * ((qa.ko != nullptr) + (qa.kc != nullptr)) + (qa.raw != nullptr ? N : 0);
-  const bool big_rows = M * row_cols * 2 > (int64_t(256) << 20);
-  const int group_m = big_rows || (tiles_n <= 4 && total >= 2048) ? 16 : 8;
+  // Row blocks per group of the tile order: an XCD has 64 workgroups resident, 16 x 4 tiles of 128 x 128 for few column
+  // blocks, once there is more than one resident round (M = 131136, N = 512, K = 1536: 230 -> 198 us for the loop alone
+  // against groups of 8; residual K = 1536 at M = 17000 / 24459 / 36000 / 60000, inputs not in cache: bf16 54.8 / 62.4 /
+  // 91.5 / 139.5 -> 50.3 / 60.4 / 86.9 / 135.0, fp32 57.5 / 70.2 / 97.9 / 150.9 -> 53.5 / 65.5 / 96.2 / 147.0, at 45057 1-2%
+  // the other way); before, 8 (M = 9000, N = 512, K = 3072: 48 -> 41 us against 16). With more column blocks:
+  //   * SwiGLU without kept rows: 16 (N = 1536 as part of an MLP, M = 9000 / 24459 / 45057 36.6 / 90.0 / 160.3 -> 35.8 /
+  //     88.1 / 156.2);
+  //   * Wqkv and SwiGLU with kept rows: 16 once the rows in and out outgrow the 256 MB last-level cache. M = 131136 with
+  //     groups of 8 and 16 (in brackets: 256 x 128 tiles in groups of 8, the same rows as 16 here): N = 1536 310 and 301 us
+  //     (305), fp32 weights and the kept product 220 and 214 (214), fp32 tables 166 and 164 (161), bf16 tables and a cache
+  //     177 and 176 (172), at M = 90000 112 and 108 (109); kept SwiGLU rows at M = 30000 / 90000 148 / 438 and 142 / 427.
+  //     Below it 8: M = 45057 97 and 98, 70 and 72, 57 and 59, 56 and 59; kept SwiGLU rows at M = 17000 84 and 95.
+  bool rows16 = false;
+  if constexpr (SH::BM == 128) {
+    int64_t row_cols = 0;
+    if constexpr (EPI == GB_QKV || EPI == GB_QKV_BF16 || EPI == GB_QKV_W32)
+      row_cols = K + 64 * qa.H + 128 * qa.HKV * ((qa.ko != nullptr) + (qa.kc != nullptr)) + (qa.raw != nullptr ? N : 0);
+    if constexpr (EPI == GB_SWIGLU) {
+      row_cols = K + 3 * static_cast<int64_t>(N);
+      rows16 = qa.raw == nullptr && total >= 2048;
+    }
+    rows16 = rows16 || M * row_cols * 2 > (int64_t(256) << 20) || (tiles_n <= 4 && total > 2 * device_cus_cached());
+  }
+  const int group_m = rows16 ? 16 : 8;
   gemm_big_kernel<EPI, SH><<<static_cast<unsigned>(total), 64 * SH::WAVES, SH::SMEM, s>>>(
       x, w, y, M, N, K, tiles_n, static_cast<int>(total), group_m, qa);
   return VK_OK;
 }
 
+template <class SH>
+static int64_t gb_tiles(int64_t M, int N) {
+  return (M + SH::BM - 1) / SH::BM * ((N + SH::BW - 1) / SH::BW);
+}
+
 template <int EPI>
 static int launch_big(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int N, int K, const GbQkv &qa,
                       hipStream_t s) {
-  // 256 x 256 tiles read a third fewer bytes into LDS per flop, but their epilogue runs alone on its CU: the faster
-  // ones only for the plain epilogues at a long K, and only where they fill the resident rounds (one workgroup per
-  // CU). N = 512, K = 3072: M = 32000 (250 tiles) 97 -> 84 us, 131136 (1026) 474 -> 442, but 45057 (354) 154 -> 160,
-  // 16000 (126) 49 -> 73; N = 512 or 1536, K = 512: 2-30% slower at every M.
-  if constexpr (EPI == GB_BF16 || EPI == GB_F32) {
-    const int64_t tiles = (M + GbWide::BM - 1) / GbWide::BM * ((N + GbWide::BW - 1) / GbWide::BW);
-    const int64_t cus = device_cus_cached(), rounds = (tiles + cus - 1) / cus;
-    if (K >= 1024 && 8 * tiles >= 7 * rounds * cus) return launch_big_shape<EPI, GbWide>(x, w, y, M, N, K, qa, s);
+  // 256 x 256 tiles read a third fewer bytes into LDS per flop, but one of them fills a CU, so its epilogue runs alone and a
+  // round of them takes 1.6-2 rounds of 128 x 128 tiles (two per CU). They are taken where their count fits its rounds the
+  // better. Plain epilogues, N = 512, bf16 out, inputs not in cache, us with 128 x 128 and 256 x 256 tiles (rounds):
+  //   K = 3072: M = 13000 (1, 1) 50, 81; 16500 (2, 1) 82, 79; 24459 (2, 1) 96, 82; 36000 (3, 2) 144, 153; 45057 (3, 2) 170, 165;
+  //   55000 (4, 2) 209, 175; 75000 (5, 3) 275, 252; 131136 (9, 5) 445, 417 (fp32 out and K = 1536 alike): from K = 1024 on
+  //   beyond one round of 128 x 128 tiles;
+  //   K = 768: 24459 28.6, 26.3; 36000 41.0, 45.7; 55000 56.4, 52.8; 75000 77, 79; 90000 (6, 3) 84.1, 81.0; 131136 124, 126:
+  //   where they halve the rounds;
+  //   K = 512: 18500 17.1, 16.6; 28000 21.4, 19.5 (fp32 out 24.1, 23.7); 55000 39.4, 39.3 (39.2, 44.8); 131136 74, 84; N =
+  //   1536: 18500 (4, 2) 34.0, 35.3; 30000 (6, 3) 52.9, 53.0: for a single round against two.
+  // The Wqkv epilogues gain only in a well-filled single round: bf16 tables and a cache, M = 15000 27.1, 28.8; 17000 30.6,
+  // 28.9; 21000 33.8, 30.8 (fp32 tables 33.0, 29.5, fp32 weights and the kept product 40.0, 39.1); not at N = 1536, M = 8000
+  // 25.7, 28.0 and 10000 29.0, 29.7.
+  const int64_t cus = device_cus_cached();
+  if constexpr (EPI == GB_BF16 || EPI == GB_F32 || EPI == GB_QKV || EPI == GB_QKV_BF16 || EPI == GB_QKV_W32) {
+    const int64_t wide = gb_tiles<GbWide>(M, N), square = gb_tiles<GbSquare>(M, N);
+    const int64_t wide_rounds = (wide + cus - 1) / cus, square_rounds = (square + 2 * cus - 1) / (2 * cus);
+    const bool fits = EPI == GB_BF16 || EPI == GB_F32
+                          ? square_rounds > 1 && (K >= 1024 || (square_rounds >= 2 * wide_rounds &&
+                                                                (K >= 768 || wide_rounds == 1)))
+                          : N <= 1024 && wide_rounds == 1 && square > 3 * cus;
+    if (fits) return launch_big_shape<EPI, GbWide>(x, w, y, M, N, K, qa, s);
   }
   // Batches whose 128 x 128 tiles leave CUs without one take smaller tiles (the same bits): a tile is a chain of slabs,
   // and more, shorter chains run side by side. Residual product N = 512, K = 512 / 1536 / 2048, us with 128 x 128, 64 x
@@ -658,13 +688,12 @@ static int launch_big(const bf16_t *x, const bf16_t *w, void *y, int64_t M, int 
   // 10.6 / 21.1 / 25.6; 9000 (284) 13.7 / 25.4 / 29.4, 11.9 / 26.6 / 30.6, 13.5 / 31.3 / 38.8. The plain and fp32
   // epilogues go the same way (N = 512, bf16 out, K = 512 / 1536 / 3072: M = 4099 6.2 / 17.3 / 32.4, 6.1 / 12.0 / 27.0, 6.1 /
   // 14.7 / 26.7; 7500 6.5 / 18.6 / 33.3, 6.3 / 17.0 / 29.9, 7.1 / 18.9 / 33.9; fp32 out, K = 512: 6.9, 6.6, 6.4 and 7.5, 7.0,
-  // 7.6); the SwiGLU product of N = 1536 has more tiles than CUs from M = 1281 on. The Wqkv epilogues keep
-  // the one shape: 64 x 128 tiles at M = 4099 take 12.5 us with bf16 tables and a cache, 10.5 with fp32 ones, 11.0 with
+  // 7.6); the SwiGLU product of N = 1536 has more tiles than CUs from M = 1281 on. The Wqkv epilogues
+  // keep 128 x 128 ones: 64 x 128 tiles at M = 4099 take 12.5 us with bf16 tables and a cache, 10.5 with fp32 ones, 11.0 with
   // fp32 weights and the kept product, 15.9 at N = 1536 without norm, against 12.4, 10.5, 12.3 and 13.9.
   if constexpr (EPI != GB_QKV && EPI != GB_QKV_BF16 && EPI != GB_QKV_W32) {
     constexpr int OUT_COLS = EPI == GB_SWIGLU ? GbSquare::BW / 2 : GbSquare::BW;
     const int64_t tiles = (M + GbSquare::BM - 1) / GbSquare::BM * ((N + OUT_COLS - 1) / OUT_COLS);
-    const int64_t cus = device_cus_cached();
     if (2 * tiles <= cus) return launch_big_shape<EPI, GbSmall>(x, w, y, M, N, K, qa, s);
     if (tiles <= cus) return launch_big_shape<EPI, GbFlat>(x, w, y, M, N, K, qa, s);
   }
