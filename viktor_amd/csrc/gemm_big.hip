@@ -628,20 +628,18 @@ static int launch_big_shape(const bf16_t *x, const bf16_t *w, void *y, int64_t M
   // the other way); before, 8 (M = 9000, N = 512, K = 3072: 48 -> 41 us against 16). With more column blocks:
   //   * SwiGLU without kept rows: 16 (N = 1536 as part of an MLP, M = 9000 / 24459 / 45057 36.6 / 90.0 / 160.3 -> 35.8 /
   //     88.1 / 156.2);
-  //   * Wqkv and SwiGLU with kept rows: 16 once the rows in and out outgrow the 256 MB last-level cache. M = 131136 with
+  //   * SwiGLU with kept rows: 8 (M = 17000 / 32772 84 / 167, with 16 95 / 179);
+  //   * Wqkv: 16 once the rows in and out outgrow the 256 MB last-level cache. M = 131136 with
   //     groups of 8 and 16 (in brackets: 256 x 128 tiles in groups of 8, the same rows as 16 here): N = 1536 310 and 301 us
   //     (305), fp32 weights and the kept product 220 and 214 (214), fp32 tables 166 and 164 (161), bf16 tables and a cache
-  //     177 and 176 (172), at M = 90000 112 and 108 (109); kept SwiGLU rows at M = 30000 / 90000 148 / 438 and 142 / 427.
-  //     Below it 8: M = 45057 97 and 98, 70 and 72, 57 and 59, 56 and 59; kept SwiGLU rows at M = 17000 84 and 95.
+  //     177 and 176 (172), at M = 90000 112 and 108 (109). Below it 8: M = 45057 97 and 98, 70 and 72, 57 and 59, 56 and
+  //     59.
   bool rows16 = false;
   if constexpr (SH::BM == 128) {
     int64_t row_cols = 0;
     if constexpr (EPI == GB_QKV || EPI == GB_QKV_BF16 || EPI == GB_QKV_W32)
       row_cols = K + 64 * qa.H + 128 * qa.HKV * ((qa.ko != nullptr) + (qa.kc != nullptr)) + (qa.raw != nullptr ? N : 0);
-    if constexpr (EPI == GB_SWIGLU) {
-      row_cols = K + 3 * static_cast<int64_t>(N);
-      rows16 = qa.raw == nullptr && total >= 2048;
-    }
+    if constexpr (EPI == GB_SWIGLU) rows16 = qa.raw == nullptr && total >= 2048;
     rows16 = rows16 || M * row_cols * 2 > (int64_t(256) << 20) || (tiles_n <= 4 && total > 2 * device_cus_cached());
   }
   const int group_m = rows16 ? 16 : 8;
