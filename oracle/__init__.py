@@ -1,7 +1,7 @@
 """CPU oracle of the decoder rollout-and-scoring path -- TEST INFRASTRUCTURE, not product code.
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may import this package, and only
-as the checker (or, for the CPU baseline, as the timed CPU restatement of the reference). The product
+to compare outputs with (or, for the CPU baseline, as the timed CPU restatement of the reference). The product
 (viktor_amd) never imports it and has no CPU fallback.
 
 oracle.reference restates, in PyTorch on the CPU:
